@@ -17,8 +17,10 @@
 // their sums in wave order. The x columns are read straight from memory: they are small and every
 // work-group reads the same ones (L2-resident after the first).
 //
-// HBM-bound: per weight 2 (F16, BF16) or 4 (F32) bytes against 1 conversion and N fused
-// multiply-adds.
+// HBM-bound at 1..2 columns: per weight 2 (F16, BF16) or 4 (F32) bytes against 1 conversion and N
+// fused multiply-adds (F16 12288x4096 17.3 / 19.2 us, 5.8 / 5.3 TB/s). At 4..8 columns the x loads
+// (2 N per 8 weight loads) and the multiply-adds count as much: 27.6 / 36 us (62.8 / 73 while the
+// sums lived in LDS, below).
 #include "kernels.h"
 
 #include <hip/hip_fp16.h>
@@ -90,23 +92,28 @@ template <> struct WLoad<BF16> {
     }
 };
 
-// reduce-scatter of V = 2^P values over the wave's 64 lanes: afterwards lane l holds, in v[0], the
-// sum over all lanes of value index_of(l)
-template <int V>
-__device__ inline void reduce_scatter(float (&v)[V], int lane) {
+// reduce-scatter of V = 2^P values over the wave's 64 lanes: lane l gets the sum over all lanes of
+// value index_of(l). A recursion over templates: written as a loop that halves its count the
+// compiler does not unroll it, indexes the sums dynamically and keeps all of them, in the main
+// loop too, in LDS (N = 8: 66 KB of it; F16 12288x4096 73 us against 36).
+template <int V, int B = 32>
+__device__ __forceinline__ float reduce_scatter(const float (&v)[V], int lane) {
+    if constexpr (V == 1) {
+        float t = v[0];
 #pragma unroll
-    for (int s = 0, n = V; n > 1; ++s, n >>= 1) {
-        const int b = 32 >> s;
-        const bool hi = (lane & b) != 0;
+        for (int b = B; b >= 1; b >>= 1) t += __shfl_xor(t, b);
+        return t;
+    } else {
+        const bool hi = (lane & B) != 0;
+        float h[V / 2];
 #pragma unroll
-        for (int i = 0; i < n / 2; ++i) {
-            const float send = hi ? v[i] : v[i + n / 2];
-            const float keep = hi ? v[i + n / 2] : v[i];
-            v[i] = keep + __shfl_xor(send, b);
+        for (int i = 0; i < V / 2; ++i) {
+            const float send = hi ? v[i] : v[i + V / 2];
+            const float keep = hi ? v[i + V / 2] : v[i];
+            h[i] = keep + __shfl_xor(send, B);
         }
+        return reduce_scatter<V / 2, B / 2>(h, lane);
     }
-#pragma unroll
-    for (int b = 32 >> __builtin_ctz(V); b >= 1; b >>= 1) v[0] += __shfl_xor(v[0], b);
 }
 
 template <int V>
@@ -128,18 +135,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NC >= 4 
     const MatArgs & a = A.a;
     const int j = A.nmat == 1 ? 0 : (tile >= A.mt[1] ? (tile >= A.mt[2] ? 2 : 1) : 0);
     const int64_t M = A.nmat > 1 ? A.Mm[j] : a.M, m0 = (tile - A.mt[j]) * kRows;
-    const int64_t i2 = sl % a.ne12, i3 = sl / a.ne12;
-    const uint8_t * w = A.nmat > 1 ? A.wm[j] : a.w + (uint64_t) (i2 / a.r2) * a.w_s2 + (uint64_t) (i3 / a.r3) * a.w_s3;
-    const float * x = a.x + i2 * a.x_s2 + i3 * a.x_s3;
-    float * yb = A.nmat > 1 ? A.ym[j] : a.y + i2 * a.y_s2 + i3 * a.y_s3;
+    const uint8_t * w = A.nmat > 1 ? A.wm[j] : a.w;
+    const float * x = a.x;
+    float * yb = A.nmat > 1 ? A.ym[j] : a.y;
     if (A.has_id) {
         // the pair's expert (read on the device, clamped into range), x column and y column
         const int64_t t = sl / A.id.n_used, i = sl - t * A.id.n_used;
         int64_t e = A.id.ids[i * A.id.s0 + t * A.id.s1];
         e = e < 0 ? 0 : (e >= A.id.n_exp ? A.id.n_exp - 1 : e);
-        w = (A.nmat > 1 ? A.wm[j] : a.w) + (uint64_t) e * a.w_s2;
-        x = a.x + (A.id.x_shared ? 0 : i) * a.x_s1 + t * a.x_s2;
-        yb = (A.nmat > 1 ? A.ym[j] : a.y) + i * a.y_s1 + t * a.y_s2;
+        w += (uint64_t) e * a.w_s2;
+        x += (A.id.x_shared ? 0 : i) * a.x_s1 + t * a.x_s2;
+        yb += i * a.y_s1 + t * a.y_s2;
+    } else if (gridDim.y > 1) { // (one slice: no 64-bit divisions ahead of the first load)
+        const int64_t i2 = sl % a.ne12, i3 = sl / a.ne12;
+        w += (uint64_t) (i2 / a.r2) * a.w_s2 + (uint64_t) (i3 / a.r3) * a.w_s3;
+        x += i2 * a.x_s2 + i3 * a.x_s3;
+        yb += i2 * a.y_s2 + i3 * a.y_s3;
     }
     const int64_t K = a.K, N = a.N;
     constexpr int esz = WT == F32 ? 4 : 2;
@@ -196,9 +207,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NC >= 4 
             }
         }
     }
-    reduce_scatter<V>(acc, lane);
+    const float part = reduce_scatter<V>(acc, lane);
     __shared__ float red[4][V];
-    red[wave][index_of<V>(lane)] = acc[0]; // (lanes holding the same index write the same sum)
+    red[wave][index_of<V>(lane)] = part; // (lanes holding the same index write the same sum)
     __syncthreads();
     const int t = threadIdx.x;
     if (t < V) {
