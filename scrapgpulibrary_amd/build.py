@@ -31,6 +31,7 @@ SOURCES = [
     ("hip/backend.cpp", ["-x", "hip"] + DEVICE),
     ("hip/matvec.hip", DEVICE),
     ("hip/matvec_float.hip", DEVICE),
+    ("hip/matmul_f32.hip", DEVICE),
     ("hip/matmul.hip", DEVICE),
     # bit-exact conversions: one IEEE operation per source operation
     ("hip/quant.hip", DEVICE + ["-ffp-contract=off"]),

@@ -72,11 +72,14 @@ struct IdArgs {
 constexpr int64_t kArriveMax = 65536;
 bool is_float_weight(int dtype);
 // float weights (launch_matvec calls it for them, launch_matmul_mfma for F32 and for K not a
-// multiple of 128): exact f32 products, K a multiple of 8, rows and slices 16-byte aligned; one
-// launch per group of 8 columns; no scratch
+// multiple of 128): exact f32 products, K a multiple of 8, rows and slices 16-byte aligned; groups
+// of 8 columns in one launch, or launch_matmul_f32 where matmul_f32_wins; no scratch
 // With `id` (N = 1): the MUL_MAT_ID pairs as launch_matvec takes them.
-hipError_t launch_matvec_float(const MatArgs * mats, int nmat, hipStream_t stream, const char ** kernel_name, uint64_t * grid_size,
+hipError_t launch_matvec_float(const MatArgs * mats, int nmat, int cu_count, hipStream_t stream, const char ** kernel_name, uint64_t * grid_size,
                                const IdArgs * id = nullptr);
+// the same products on the f32 matrix units (F32: more than 8 columns)
+hipError_t launch_matmul_f32(const MatArgs * mats, int nmat, int cu_count, hipStream_t stream, const char ** kernel_name, uint64_t * grid_size);
+bool matmul_f32_wins(const MatArgs * mats, int nmat, int cu_count);
 size_t matvec_scratch_bytes(const MatArgs * mats, int nmat, const IdArgs * id = nullptr);
 hipError_t launch_matvec(const MatArgs * mats, int nmat, int cu_count, hipStream_t stream, const char ** kernel_name,
                          uint64_t * grid_size, const IdArgs * id = nullptr, uint8_t * scratch = nullptr, uint32_t * arrive = nullptr);

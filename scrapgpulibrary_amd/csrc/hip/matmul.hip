@@ -2214,7 +2214,7 @@ hipError_t launch_matmul_mfma(const MatArgs * mats, int nmat, uint8_t * scratch,
         if (mats[j].dtype != a.dtype || !matmul_reads_same_x(mats[j], a) || mats[j].ne12 * mats[j].ne13 != 1 || a.ne12 * a.ne13 != 1) return hipErrorInvalidValue;
         a.M += mats[j].M;
     }
-    if (is_float_weight(a.dtype) && !float_gemm(a)) return launch_matvec_float(mats, nmat, stream, kernel_name, nullptr);
+    if (is_float_weight(a.dtype) && !float_gemm(a)) return launch_matvec_float(mats, nmat, cu_count, stream, kernel_name, nullptr);
     uint16_t * xb = reinterpret_cast<uint16_t *>(scratch);
     const int64_t rows = a.N * a.ne12 * a.ne13;
     float * xs = reinterpret_cast<float *>(scratch + xs_offset(a));

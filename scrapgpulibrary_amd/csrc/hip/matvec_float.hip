@@ -1,5 +1,5 @@
 // Decode matvec over float weights (F32 / F16 / BF16 rows in the natural layout) for 1 <= N <= 8
-// columns (gfx950, wave64).
+// columns, or more in groups of 8 (gfx950, wave64).
 //
 // Replaces, for the hip backend, the reference's float-weight matvec kernels (the F32 / F16 arms
 // of src/backends/opencl11/ops_matmul.cpp:67-123, kernels/mul_mv.cl) with the product of the CPU
@@ -20,10 +20,9 @@
 // HBM-bound at 1..2 columns: per weight 2 (F16, BF16) or 4 (F32) bytes against 1 conversion and N
 // fused multiply-adds (F16 12288x4096 17.3 / 19.2 us, 5.8 / 5.3 TB/s). At 4..8 columns the x loads
 // (2 N per 8 weight loads) and the multiply-adds count as much: 27.6 / 36 us (62.8 / 73 while the
-// sums lived in LDS, below).
+// sums lived in LDS, below); matmul_f32.hip takes the large F16 / BF16 products there.
 #include "kernels.h"
-
-#include <hip/hip_fp16.h>
+#include "weight_float.h"
 
 #include <algorithm>
 #include <cstdio>
@@ -45,51 +44,6 @@ struct MvfArgs {
     int64_t ys1m[3];
     IdArgs id;     // MUL_MAT_ID (has_id): blockIdx.y is the pair t * n_used + i
     int has_id;
-};
-
-// 16 bytes of weights, non-temporal (read once per product, as in the quantized matvec)
-typedef unsigned int u32x4_nt __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint4 ld16_nt(const uint8_t * p) {
-    const u32x4_nt v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_nt *>(p));
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-
-// 8 consecutive weights of one row as f32 (p 16-byte aligned)
-template <int WT> struct WLoad;
-template <> struct WLoad<F32> {
-    uint4 u, v;
-    __device__ void load(const uint8_t * p) {
-        u = ld16_nt(p);
-        v = ld16_nt(p + 16);
-    }
-    __device__ void to_f32(float * o) const {
-        o[0] = __uint_as_float(u.x), o[1] = __uint_as_float(u.y), o[2] = __uint_as_float(u.z), o[3] = __uint_as_float(u.w);
-        o[4] = __uint_as_float(v.x), o[5] = __uint_as_float(v.y), o[6] = __uint_as_float(v.z), o[7] = __uint_as_float(v.w);
-    }
-};
-template <> struct WLoad<F16> {
-    uint4 q;
-    __device__ void load(const uint8_t * p) { q = ld16_nt(p); }
-    __device__ void to_f32(float * o) const {
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[2 * i] = __half2float(__ushort_as_half((unsigned short) (w[i] & 0xFFFFu)));
-            o[2 * i + 1] = __half2float(__ushort_as_half((unsigned short) (w[i] >> 16)));
-        }
-    }
-};
-template <> struct WLoad<BF16> {
-    uint4 q;
-    __device__ void load(const uint8_t * p) { q = ld16_nt(p); }
-    __device__ void to_f32(float * o) const {
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[2 * i] = __uint_as_float(w[i] << 16);
-            o[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-        }
-    }
 };
 
 // reduce-scatter of V = 2^P values over the wave's 64 lanes: lane l gets the sum over all lanes of
@@ -152,7 +106,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NC >= 4 
         x += i2 * a.x_s2 + i3 * a.x_s3;
         yb += i2 * a.y_s2 + i3 * a.y_s3;
     }
-    const int64_t K = a.K, N = a.N;
+    const int64_t n0 = (int64_t) blockIdx.z * NC; // (a column group)
+    const int64_t K = a.K, N = a.N - n0;
+    x += n0 * a.x_s1;
     constexpr int esz = WT == F32 ? 4 : 2;
     const uint8_t * row[kRows];
 #pragma unroll
@@ -217,7 +173,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NC >= 4 
         const float sum = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
         if (m0 + r < M && c < N) {
             const int64_t ys1 = A.nmat > 1 ? A.ys1m[j] : a.y_s1;
-            yb[c * ys1 + m0 + r] = sum; // (MUL_MAT_ID: one column)
+            yb[(n0 + c) * ys1 + m0 + r] = sum; // (MUL_MAT_ID: one column)
         }
     }
 }
@@ -238,26 +194,12 @@ bool is_float_weight(int dtype) {
     return dtype == F32 || dtype == F16 || dtype == BF16;
 }
 
-hipError_t launch_matvec_float(const MatArgs * mats, int nmat, hipStream_t stream, const char ** kernel_name, uint64_t * grid_size,
+hipError_t launch_matvec_float(const MatArgs * mats, int nmat, int cu_count, hipStream_t stream, const char ** kernel_name, uint64_t * grid_size,
                                const IdArgs * id) {
     if (nmat < 1 || nmat > 3) return hipErrorInvalidValue;
     if (id != nullptr && (mats[0].N != 1 || id->ids == nullptr || id->n_used < 1 || id->n_tok < 1 || id->n_exp < 1)) return hipErrorInvalidValue;
-    if (mats[0].N > 8 && id == nullptr) {
-        // more columns (F32 weights, or K not a whole number of GEMM stages): one launch per group
-        // of 8 columns, each the exact product above
-        for (int64_t c0 = 0; c0 < mats[0].N; c0 += 8) {
-            MatArgs g[3];
-            for (int j = 0; j < nmat; ++j) {
-                g[j] = mats[j];
-                g[j].N = std::min<int64_t>(8, mats[j].N - c0);
-                g[j].x = mats[j].x + c0 * mats[j].x_s1;
-                g[j].y = mats[j].y + c0 * mats[j].y_s1;
-            }
-            const hipError_t e = launch_matvec_float(g, nmat, stream, kernel_name, grid_size);
-            if (e != hipSuccess) return e;
-        }
-        std::snprintf(last_form().form, sizeof(last_form().form), "float rows=8 column-groups=%d", (int) ((mats[0].N + 7) / 8));
-        return hipSuccess;
+    if (id == nullptr && is_float_weight(mats[0].dtype) && matmul_f32_wins(mats, nmat, cu_count)) {
+        return launch_matmul_f32(mats, nmat, cu_count, stream, kernel_name, grid_size);
     }
     const MatArgs & a = mats[0];
     if (!is_float_weight(a.dtype) || a.N < 1 || a.K < 8 || a.K % 8 != 0) return hipErrorInvalidValue;
@@ -283,17 +225,30 @@ hipError_t launch_matvec_float(const MatArgs * mats, int nmat, hipStream_t strea
     }
     const int64_t slices = id != nullptr ? id->n_used * id->n_tok : a.ne12 * a.ne13;
     if (A.mt[nmat] > 0x7fffffff || slices > 65535) return hipErrorInvalidValue;
-    const int nc = (int) a.N;
+    // more than 8 columns (F32 weights, or K not a whole number of GEMM stages): groups of 8 on
+    // blockIdx.z, one launch (F32 128x2048 at 37 columns 6.4 us against 32.6 in 5 launches)
+    const int nc = (int) std::min<int64_t>(a.N, 8);
+    const int64_t groups = (a.N + 7) / 8, per = 65535;
     const bool xv = (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && a.x_s1 % 4 == 0 && a.x_s2 % 4 == 0 && a.x_s3 % 4 == 0;
     void * fn = a.dtype == F32 ? kernel_for<F32>(nc, xv) : a.dtype == F16 ? kernel_for<F16>(nc, xv) : kernel_for<BF16>(nc, xv);
     const int ncp = nc == 1 ? 1 : nc == 2 ? 2 : nc <= 4 ? 4 : 8;
-    const dim3 grid((unsigned) A.mt[nmat], (unsigned) slices);
-    void * args[] = {&A};
     if (kernel_name) *kernel_name = a.dtype == F32 ? "matvec_f32" : a.dtype == F16 ? "matvec_f16" : "matvec_bf16";
-    std::snprintf(last_form().form, sizeof(last_form().form), "float rows=%d nc=%d", kRows, ncp);
-    last_form().grid = (uint64_t) grid.x * grid.y;
+    if (groups > 1) std::snprintf(last_form().form, sizeof(last_form().form), "float rows=%d column-groups=%d", kRows, (int) groups);
+    else std::snprintf(last_form().form, sizeof(last_form().form), "float rows=%d nc=%d", kRows, ncp);
+    last_form().grid = (uint64_t) A.mt[nmat] * (uint64_t) slices * (uint64_t) groups;
     if (grid_size) *grid_size = last_form().grid;
-    return hipLaunchKernel(fn, grid, dim3(256), args, 0, stream);
+    for (int64_t g0 = 0; g0 < groups; g0 += per) {
+        const int64_t c0 = 8 * g0;
+        A.a.N = std::min<int64_t>(8 * per, a.N - c0);
+        A.a.x = a.x + c0 * a.x_s1;
+        A.a.y = a.y + c0 * a.y_s1;
+        for (int j = 0; j < nmat; ++j) A.ym[j] = mats[j].y + c0 * mats[j].y_s1;
+        const dim3 grid((unsigned) A.mt[nmat], (unsigned) slices, (unsigned) std::min<int64_t>(per, groups - g0));
+        void * args[] = {&A};
+        const hipError_t e = hipLaunchKernel(fn, grid, dim3(256), args, 0, stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 } // namespace sgk
