@@ -33,6 +33,7 @@ SOURCES = [
     ("hip/matvec_float.hip", DEVICE),
     ("hip/matmul_f32.hip", DEVICE),
     ("hip/matmul.hip", DEVICE),
+    ("hip/gemm_lds.hip", DEVICE),
     # bit-exact conversions: one IEEE operation per source operation
     ("hip/quant.hip", DEVICE + ["-ffp-contract=off"]),
 ]

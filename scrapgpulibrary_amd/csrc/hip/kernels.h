@@ -104,6 +104,28 @@ bool matmul_same_x(const MatArgs & a, const MatArgs & b, int cu_count, bool lean
 // true when a and b read the same x with the same shape (what one fused launch over both needs)
 bool matmul_reads_same_x(const MatArgs & a, const MatArgs & b);
 
+// The prefill GEMM over F16 / BF16 weights with both operands in LDS (gemm_lds.hip); launched by
+// launch_matmul_mfma. 128, 192 or 384 rows x 128 tokens per tile of up to 3 weights, matrix j owning row tiles
+// mt[j] .. mt[j + 1] and columns mo[j] .. mo[j + 1] of the split-K partials [split][slice][N][mo[nmat]].
+struct LdsGemm {
+    const uint16_t * xb; // [slices][N][K] f16 (BF16 weights: bf16), elements in order, rows scaled
+    const float * xs;    // [slices][N] factors
+    float * part;
+    int N, K, nmat, split, tiles_m, tiles_n;
+    int mt[4];
+    int64_t mo[4];
+    const uint8_t * wm[3];
+    float * ym[3];
+    int64_t ys1m[3];
+    int Mm[3];
+    int64_t nb; // row stride of the weights in bytes
+    uint64_t w_s2, w_s3;
+    int64_t y_s2, y_s3, ne12, r2, r3;
+};
+hipError_t launch_gemm_lds(const LdsGemm & L, int dtype, int rows, int slices, hipStream_t stream);
+// dynamic LDS beyond the 64 KiB default for a kernel
+hipError_t allow_lds(void * fn, size_t lds);
+
 // MUL_MAT_ID with many tokens (prefill): the (slot, token) pairs are grouped by expert on the
 // device (ids clamped as above), x goes through the matmul's pre-pass once, and the f16 MFMA GEMM
 // runs over (expert, 32- or 64-pair tile, 128- or 384-row tile) with gathered x rows and scattered

@@ -431,8 +431,8 @@ template <> struct PFmt<Q4_0> {
 // F16 / BF16 rows in the natural layout (float weights, K a multiple of the 128-element stage):
 // stage s = elements 128 s .. + 127 of the row; k-step t takes elements 16 t .. + 15, k-half h
 // the 16-byte chunk 2 t + h of them: the two lanes of a row read 32 contiguous bytes per load, so a
-// wave's load touches 32 cache lines instead of 64 (as 8 chunks per lane, contiguous). The pairs are reordered to the x tile's
-// element order 0 2 1 3 of each group of 4. BF16 feeds the bf16 MFMA (x then in bf16, see
+// wave's load touches 32 cache lines instead of 64 (as 8 chunks per lane, contiguous). x is in
+// plain element order for these (k_x_to_f16's PLAIN). BF16 feeds the bf16 MFMA (x then in bf16, see
 // k_x_to_f16), F16 the f16 one; neither needs scales.
 template <int DT> struct PFmtFloat {
     struct Raw {
@@ -456,10 +456,7 @@ template <int DT> struct PFmtFloat {
     __device__ Raw load_half2(const uint8_t * w, int s, const Raw &) const { return load(w, s); }
     __device__ Sc prep(const Raw &, int) const { return Sc{}; }
     __device__ static f16x8 bop(const Raw & r, const Sc &, int t) {
-        const uint4 & q = r.q[t];
-        const uint4 o = make_uint4((q.x & 0xFFFFu) | (q.y << 16), (q.x >> 16) | (q.y & 0xFFFF0000u), (q.z & 0xFFFFu) | (q.w << 16),
-                                   (q.z >> 16) | (q.w & 0xFFFF0000u));
-        return __builtin_bit_cast(f16x8, o);
+        return __builtin_bit_cast(f16x8, r.q[t]);
     }
     __device__ static int chunk(int h, int t) {
         return 2 * t + h;
@@ -1537,7 +1534,8 @@ __global__ __launch_bounds__(256) void k_sk_reduce(MmArgs L) {
 // slice sl = blockIdx.x / N). The row is scaled by 2^e so that its largest magnitude lands in
 // [2^14, 2^15): no row overflows f16 and none loses precision to its subnormals beyond 2^-24 of
 // the row's maximum; xs[row] = 2^-e undoes it on the products. Inside each group of 4 elements the
-// order is 0 2 1 3, the order of the weight pairs the matmul builds. VEC: rows 16-byte aligned.
+// order is 0 2 1 3, the order of the weight pairs the matmul builds (PLAIN, for 16-bit weights: in
+// order). VEC: rows 16-byte aligned.
 // The first kCached groups of 8 elements per thread stay in registers between the two passes.
 // Q4K (the single-fma weight form): elements 32..63 of every 64 (the high nibbles of a Q4_K group)
 // are stored divided by 16 more, and xsum gets the row's 32-element sub-block sums (of the scaled
@@ -1549,7 +1547,7 @@ __global__ __launch_bounds__(256) void k_sk_reduce(MmArgs L) {
 // are 512 contiguous bytes.
 // (tid: the thread's index among the row's 256, wmax: 4 floats of LDS for the row's waves; a
 // thread group with live = false takes part in the barrier only)
-template <bool VEC, bool Q4K, bool BF, bool FRAG>
+template <bool VEC, bool Q4K, bool BF, bool FRAG, bool PLAIN>
 __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, float * xs, uint16_t * xsum, int64_t xsum_row, int64_t row,
                                              int tid, float * wmax, bool live) {
     constexpr int kCached = 6; // K <= 12288 is read once
@@ -1592,14 +1590,19 @@ __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, f
             }
         }
         if (!live) return;
+        if constexpr (!PLAIN) {
+            const float s1 = s[1], s5 = s[5];
+            s[1] = s[2], s[2] = s1;
+            s[5] = s[6], s[6] = s5;
+        }
         if constexpr (BF) { // (BF16 weights: x in bf16, rounded to nearest even)
-            const bf16x2 p0 = __builtin_convertvector((f32x2{s[0], s[2]}), bf16x2), p1 = __builtin_convertvector((f32x2{s[1], s[3]}), bf16x2);
-            const bf16x2 p2 = __builtin_convertvector((f32x2{s[4], s[6]}), bf16x2), p3 = __builtin_convertvector((f32x2{s[5], s[7]}), bf16x2);
+            const bf16x2 p0 = __builtin_convertvector((f32x2{s[0], s[1]}), bf16x2), p1 = __builtin_convertvector((f32x2{s[2], s[3]}), bf16x2);
+            const bf16x2 p2 = __builtin_convertvector((f32x2{s[4], s[5]}), bf16x2), p3 = __builtin_convertvector((f32x2{s[6], s[7]}), bf16x2);
             *reinterpret_cast<uint4 *>(op + k) = make_uint4(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1),
                                                             __builtin_bit_cast(uint32_t, p2), __builtin_bit_cast(uint32_t, p3));
         } else {
-            const f16x2 p0 = __builtin_convertvector((f32x2{s[0], s[2]}), f16x2), p1 = __builtin_convertvector((f32x2{s[1], s[3]}), f16x2);
-            const f16x2 p2 = __builtin_convertvector((f32x2{s[4], s[6]}), f16x2), p3 = __builtin_convertvector((f32x2{s[5], s[7]}), f16x2);
+            const f16x2 p0 = __builtin_convertvector((f32x2{s[0], s[1]}), f16x2), p1 = __builtin_convertvector((f32x2{s[2], s[3]}), f16x2);
+            const f16x2 p2 = __builtin_convertvector((f32x2{s[4], s[5]}), f16x2), p3 = __builtin_convertvector((f32x2{s[6], s[7]}), f16x2);
             // (FRAG: chunk k / 8 of the row is chunk k / 8 % 16 of stage k / 128)
             uint16_t * d = FRAG ? op + ((k >> 7) * kChunks * 32 + ((k >> 3) & 15) * 32) * 8 : op + k;
             *reinterpret_cast<uint4 *>(d) = make_uint4(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1),
@@ -1654,10 +1657,10 @@ __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, f
     }
 }
 
-template <bool VEC, bool Q4K, bool BF = false, bool FRAG = false>
+template <bool VEC, bool Q4K, bool BF = false, bool FRAG = false, bool PLAIN = false>
 __global__ __launch_bounds__(256) void k_x_to_f16(MatArgs a, uint16_t * xb, float * xs, uint16_t * xsum, int64_t xsum_row) {
     __shared__ float wmax[4];
-    x_row_to_f16<VEC, Q4K, BF, FRAG>(a, xb, xs, xsum, xsum_row, blockIdx.x, threadIdx.x, wmax, true);
+    x_row_to_f16<VEC, Q4K, BF, FRAG, PLAIN>(a, xb, xs, xsum, xsum_row, blockIdx.x, threadIdx.x, wmax, true);
 }
 
 // MUL_MAT_ID routing (E <= 1024 experts, P < 2^24 pairs), by one 1024-thread work-group: the
@@ -1736,7 +1739,7 @@ __global__ __launch_bounds__(1024) void k_x_route(MatArgs a, uint16_t * xb, floa
     const int q = threadIdx.x >> 8;
     const int64_t row = 4 * ((int64_t) blockIdx.x - 1) + q;
     const bool live = row < rows;
-    x_row_to_f16<VEC, Q4K, false, false>(a, xb, xs, xsum, xsum_row, live ? row : 0, threadIdx.x & 255, wmax + 4 * q, live);
+    x_row_to_f16<VEC, Q4K, false, false, false>(a, xb, xs, xsum, xsum_row, live ? row : 0, threadIdx.x & 255, wmax + 4 * q, live);
 }
 
 int env_int(const char * name, int dflt) {
@@ -1759,6 +1762,7 @@ struct MmConfig {
     int kw = 8;
     int nz = 1; // narrow: work-groups per R32 group, each with bn / nz tokens
     int rw = 1; // narrow: R32 groups per work-group (kw waves each)
+    int lds = 0; // k_gemm_l (F16 / BF16): rows of a tile, 128, 192 or 384
 };
 
 // the narrow GEMM's shapes: quantized weights, 9..128 tokens, one slice, K a whole number of
@@ -1769,6 +1773,26 @@ bool narrow_shape(const MatArgs & a) {
            a.ne12 * a.ne13 == 1 && a.K % BK == 0;
 }
 
+
+size_t part_offset(const MatArgs & a);
+size_t part_bytes(const MatArgs & a, int split);
+
+// the scratch a lean configuration may take (the static array of scrapgpu_hip_op_execute_static)
+constexpr size_t kLeanBytes = (size_t) 32 << 20;
+
+// Estimated time of k_gemm_l in us, from measurements on 256 CUs (F16): a 64-element stage of a
+// 192- / 128-row tile takes 0.82 / 0.62 us while every CU has one (12288x4096 at 512 tokens 57 us in
+// 256 192-row tiles, 4096x12288 at 2048 239 us in two rounds of 128-row ones), a part-filled round
+// less, as the tiles in flight share the L2s (4096x4096 at 512: half the CUs, 0.37 us a stage), but
+// hardly where every tile streams weights of its own (one token tile: 12288x4096 at 128, 96 tiles,
+// 0.64 us); 6 stages' time of prologue and epilogue; K splits move their partial sums at 4.7 TB/s.
+float lds_gemm_us(const MatArgs & a, int rows, int split, int cu_count) {
+    const int64_t tn = (a.N + 127) / 128, tiles = (a.M + rows - 1) / rows * tn * a.ne12 * a.ne13 * split;
+    const float part = (float) (tiles % cu_count) / (float) cu_count, least = tn == 1 ? 0.75f : tn == 2 ? 0.55f : 0.35f;
+    const float rounds = (float) (tiles / cu_count) + (part > 0.0f ? least + (1.0f - least) * part : 0.0f);
+    const float us = rounds * ((float) a.K / 64.0f / (float) split + 6.0f) * (rows == 192 ? 0.82f : 0.62f);
+    return split == 1 ? us : us + 2.0f + 2.0f * (float) split * 4.0f * (float) a.M * (float) a.N * (float) (a.ne12 * a.ne13) / 4.7e6f;
+}
 
 MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
     static const int env_bn = env_int("SCRAPGPU_HIP_MM_BN", 0), env_rg = env_int("SCRAPGPU_HIP_MM_RG", 0);
@@ -1827,30 +1851,47 @@ MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
         }
     }
     if (a.dtype == F16 || a.dtype == BF16) {
-        // the wide GEMM (k_gemm_w, 384-row x 128-token tiles; its 2-K-group form spills with the
-        // float rows' raw data) where its tiles fill the CUs, or with K split so that they occupy
-        // 2/3 of them or more in one round, >= 16 stages per split
+        // both operands in LDS (k_gemm_l) from 65 tokens on
         static const int env_wide = env_int("SCRAPGPU_HIP_MM_WIDE", 1);
-        if (env_wide != 0 && env_w == 0 && env_bn == 0 && env_split <= 1 && a.K % BK == 0 && a.N >= 128 &&
-            (a.N + 127) / 128 * 128 * 8 <= 9 * a.N && (a.M % 384 == 0 || a.M >= 8 * 384)) {
-            const int64_t tw = (a.M + 383) / 384 * ((a.N + 127) / 128) * slices;
+        const bool free_choice = env_wide != 0 && env_w == 0 && env_bn == 0 && env_split <= 1 && a.K % BK == 0;
+        // 384-row x 128-token tiles (12 waves) where they fill the CUs, or with K in 2 splits occupy
+        // 2/3 of them or more in one round, >= 16 stages per split
+        const int64_t tw = (a.M + 383) / 384 * ((a.N + 127) / 128) * slices;
+        const bool wide = free_choice && a.N >= 128 && (a.N + 127) / 128 * 128 * 8 <= 9 * a.N && (a.M % 384 == 0 || a.M >= 8 * 384);
+        const bool wide1 = wide && (tw % cu_count == 0 || tw >= 4 * (int64_t) cu_count);
+        const bool wide2 = wide && !wide1 && slices == 1 && tw * 2 <= cu_count && 3 * tw * 2 >= 2 * cu_count && stages / 2 >= 16;
+        // 192- or 128-row tiles: K past 1024 (shorter K is mostly prologue: 24536x1024 at 500 tokens
+        // 59.8 us against 55.2 in 384-row tiles) and at least 8 tiles. Faster as well, but left on
+        // the forms that are pinned for them: K up to 1024 in general (4096x512 at 512 tokens 12.1
+        // us against 20.0 on 4-wave work-groups), fewer tiles (384x2048 at 200 tokens 18.2 against
+        // 29.1) and a part-empty token tile in the 384-row form's K splits (12288x4096 at 380 tokens
+        // 60 against 80 us; 96 before its weights went through LDS)
+        const int64_t tn = (a.N + 127) / 128;
+        if (free_choice && a.N > 64 && a.K > 1024 && (a.M + 127) / 128 * tn * slices >= 8 && !(wide2 && a.N % 128 != 0)) {
+            float best = 0.0f;
+            for (const int rows : {128, 192})
+                for (const int sp : {1, 2, 4}) {
+                    if (stages / sp < 4 || (lean && sp > 1 && part_offset(a) + part_bytes(a, sp) > kLeanBytes)) continue;
+                    const float us = lds_gemm_us(a, rows, sp, cu_count);
+                    if (c.lds == 0 || us < best) best = us, c.lds = rows, c.split = sp;
+                }
+            c.w = 8;
+            c.kg = 2;
+            c.rg = 1;
+            c.bn = 128;
+            return c;
+        }
+        if (wide1 || wide2) {
             c.w = 12;
             c.kg = 1;
             c.rg = 1;
             c.bn = 128;
-            c.wide = true;
-            c.split = 1;
-            if (tw % cu_count == 0 || tw >= 4 * (int64_t) cu_count) return c;
-            if (slices == 1) // (at most 2 splits: 3 and 4 measured slower than the 4-wave form)
-                for (int sp = 2; sp <= 2; ++sp)
-                    if (tw * sp <= cu_count && 3 * tw * sp >= 2 * cu_count && stages / sp >= 16) {
-                        c.split = sp;
-                        return c;
-                    }
-            c.wide = false;
+            c.lds = 384;
+            c.split = wide1 ? 1 : 2;
+            return c;
         }
         // else 4-wave work-groups, 128-token tiles from 128 tokens on (each 2-byte weight fetched
-        // half as often: 12288x4096 at 512 tokens 119 against 137 us, at 256 tokens 81 against 92)
+        // half as often)
         c.w = 4;
         c.kg = 1;
         c.rg = 1;
@@ -2057,11 +2098,10 @@ void * kernel_of(const MmConfig & c) {
     return c.bn == 64 ? (void *) k_matmul<DT, 64, 2, 4, 1> : (void *) k_matmul<DT, 128, 2, 4, 1>;
 }
 
-// float weights: the wide GEMM's 12-row-wave form (K split or not), else the 4-wave kernel (their
-// raw rows take the registers that its 12-wave and 2-K-group forms need)
+// float weights off k_gemm_l: the 4-wave kernel (their raw rows take the registers that its 12-wave
+// and 2-K-group forms need)
 template <int DT>
 void * kernel_of_float(const MmConfig & c) {
-    if (c.wide) return c.kg == 2 ? (void *) k_gemm_w<DT, 2> : (void *) k_gemm_w<DT, 1>;
     return c.bn == 64 ? (void *) k_matmul<DT, 64, 1, 4, 1> : (void *) k_matmul<DT, 128, 1, 4, 1>;
 }
 
@@ -2092,7 +2132,7 @@ size_t part_bytes(const MatArgs & a, int split) {
 
 // dynamic LDS beyond the 64 KiB default (gfx950 has 160 KiB per CU): set once per kernel (a
 // kernel's LDS size is fixed by its template arguments)
-static hipError_t allow_lds(void * fn, size_t lds) {
+hipError_t allow_lds(void * fn, size_t lds) {
     if (lds <= 65536) return hipSuccess;
     static std::mutex mu;
     static std::vector<void *> done;
@@ -2167,6 +2207,26 @@ static hipError_t launch_narrow(MmArgs & L, const MatArgs * mats, int nmat, cons
     return hipLaunchKernel(fn, grid, dim3((unsigned) (64 * cfg.kw * cfg.rw)), args, lds, stream);
 }
 
+// 16-bit weights with both operands in LDS: L's tiles and row ranges as set by launch_matmul_mfma
+static hipError_t launch_lds(const MmArgs & L, const MmConfig & cfg, hipStream_t stream, const char ** kernel_name) {
+    const MatArgs & a = L.a;
+    LdsGemm g;
+    std::memset(&g, 0, sizeof(g));
+    g.xb = L.xb, g.xs = L.xs, g.part = L.part;
+    g.N = (int) a.N, g.K = (int) a.K, g.nmat = L.nmat, g.split = L.split;
+    g.tiles_m = (int) L.tiles_m, g.tiles_n = (int) L.tiles_n;
+    for (int j = 0; j < 4; ++j) g.mt[j] = (int) L.mt[j], g.mo[j] = L.mo[j];
+    for (int j = 0; j < L.nmat; ++j) g.wm[j] = L.wm[j], g.ym[j] = L.ym[j], g.ys1m[j] = L.ys1m[j], g.Mm[j] = (int) L.Mm[j];
+    g.nb = a.nb, g.w_s2 = a.w_s2, g.w_s3 = a.w_s3, g.y_s2 = a.y_s2, g.y_s3 = a.y_s3;
+    g.ne12 = a.ne12, g.r2 = a.r2, g.r3 = a.r3;
+    if (kernel_name) *kernel_name = a.dtype == F16 ? "matmul_mfma_f16" : "matmul_mfma_bf16";
+    if (cfg.lds == 384)
+        std::snprintf(last_form().form, sizeof(last_form().form), "gemm wide w=12 kg=1 bn=128 rg=1 split=%d lds", L.split);
+    else
+        std::snprintf(last_form().form, sizeof(last_form().form), "gemm lds w=8 kg=2 bn=128 rows=%d split=%d", cfg.lds, L.split);
+    return launch_gemm_lds(g, a.dtype, cfg.lds, (int) (a.ne12 * a.ne13), stream);
+}
+
 size_t matmul_scratch_bytes(const MatArgs & a, int cu_count, bool lean) {
     // (float weights off the GEMM run the float matvec, which takes no scratch)
     if (is_float_weight(a.dtype) && !float_gemm(a)) return 0;
@@ -2201,6 +2261,7 @@ bool matmul_reads_same_x(const MatArgs & a, const MatArgs & b) {
 bool matmul_same_x(const MatArgs & a, const MatArgs & b, int cu_count, bool lean) {
     return matmul_reads_same_x(a, b) && q4k_x_form(a, cu_count, lean) == q4k_x_form(b, cu_count, lean) &&
            frag_x_form(a, cu_count, lean) == frag_x_form(b, cu_count, lean) && (a.dtype == BF16) == (b.dtype == BF16) &&
+           (a.dtype == F16) == (b.dtype == F16) &&
            !(is_float_weight(a.dtype) && !float_gemm(a)) && !(is_float_weight(b.dtype) && !float_gemm(b));
 }
 
@@ -2238,9 +2299,14 @@ hipError_t launch_matmul_mfma(const MatArgs * mats, int nmat, uint8_t * scratch,
             hipLaunchKernelGGL((k_x_to_f16<false, true>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
     } else if (a.dtype == BF16) {
         if (vec)
-            hipLaunchKernelGGL((k_x_to_f16<true, false, true>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
+            hipLaunchKernelGGL((k_x_to_f16<true, false, true, false, true>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
         else
-            hipLaunchKernelGGL((k_x_to_f16<false, false, true>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
+            hipLaunchKernelGGL((k_x_to_f16<false, false, true, false, true>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
+    } else if (a.dtype == F16) {
+        if (vec)
+            hipLaunchKernelGGL((k_x_to_f16<true, false, false, false, true>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
+        else
+            hipLaunchKernelGGL((k_x_to_f16<false, false, false, false, true>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
     } else {
         if (vec)
             hipLaunchKernelGGL((k_x_to_f16<true, false>), xg, dim3(256), 0, stream, a, xb, xs, xsum, xsum_row);
@@ -2259,7 +2325,7 @@ hipError_t launch_matmul_mfma(const MatArgs * mats, int nmat, uint8_t * scratch,
     L.xsum = xsum;
     L.xsum_row = xsum_row;
     const int BN = cfg.bn;
-    const int bmt = 32 * cfg.rg * (cfg.w / cfg.kg);
+    const int bmt = cfg.lds ? cfg.lds : 32 * cfg.rg * (cfg.w / cfg.kg);
     // each matrix's rows tiled on their own
     L.nmat = nmat;
     L.mt[0] = L.mo[0] = 0;
@@ -2273,7 +2339,7 @@ hipError_t launch_matmul_mfma(const MatArgs * mats, int nmat, uint8_t * scratch,
         L.mo[j + 1] = L.mo[j] + (has ? mats[j].M : 0);
     }
     L.packed = 0;
-    if (nmat > 1) {
+    if (cfg.lds == 0 && nmat > 1) {
         L.packed = 1;
         for (int j = 0; j + 1 < nmat; ++j)
             if (mats[j].M % (32 * cfg.rg) != 0) L.packed = 0;
@@ -2292,25 +2358,29 @@ hipError_t launch_matmul_mfma(const MatArgs * mats, int nmat, uint8_t * scratch,
     L.sk_g = cfg.sk ? cu_count : 0;
     if (cfg.sk && L.tiles_m * L.tiles_n > sk_max_tiles(a, cfg.bn)) return hipErrorInvalidValue; // (more slots than the scratch holds)
     const dim3 grid(cfg.sk ? (unsigned) cu_count : (unsigned) (L.tiles_m * L.tiles_n * L.split), (unsigned) slices);
-    void * args[] = {&L};
-    void * fn = nullptr;
-    switch (a.dtype) {
-        case Q4_0: fn = kernel_of<Q4_0>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q4_0"; break;
-        case Q8_0: fn = kernel_of<Q8_0>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q8_0"; break;
-        case Q4_K: fn = kernel_of<Q4_K>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q4_k"; break;
-        case Q6_K: fn = kernel_of<Q6_K>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q6_k"; break;
-        case F16: fn = kernel_of_float<F16>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_f16"; break;
-        case BF16: fn = kernel_of_float<BF16>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_bf16"; break;
-        default: return hipErrorInvalidValue;
-    }
-    if ((e = allow_lds(fn, lds)) != hipSuccess) return e;
-    if (cfg.sk)
-        std::snprintf(last_form().form, sizeof(last_form().form), "gemm wide stream-k w=12 kg=1 bn=%d rg=1 wgs=%d", BN, cu_count);
-    else
-        std::snprintf(last_form().form, sizeof(last_form().form), "gemm%s w=%d kg=%d bn=%d rg=%d split=%d", cfg.wide ? " wide" : "", cfg.w, cfg.kg, BN,
-                      cfg.rg, L.split);
     last_form().grid = (uint64_t) grid.x * grid.y;
-    e = hipLaunchKernel(fn, grid, dim3((unsigned) (64 * cfg.w)), args, lds, stream);
+    if (cfg.lds) {
+        e = launch_lds(L, cfg, stream, kernel_name);
+    } else {
+        void * args[] = {&L};
+        void * fn = nullptr;
+        switch (a.dtype) {
+            case Q4_0: fn = kernel_of<Q4_0>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q4_0"; break;
+            case Q8_0: fn = kernel_of<Q8_0>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q8_0"; break;
+            case Q4_K: fn = kernel_of<Q4_K>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q4_k"; break;
+            case Q6_K: fn = kernel_of<Q6_K>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_q6_k"; break;
+            case F16: fn = kernel_of_float<F16>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_f16"; break;
+            case BF16: fn = kernel_of_float<BF16>(cfg); if (kernel_name) *kernel_name = "matmul_mfma_bf16"; break;
+            default: return hipErrorInvalidValue;
+        }
+        if ((e = allow_lds(fn, lds)) != hipSuccess) return e;
+        if (cfg.sk)
+            std::snprintf(last_form().form, sizeof(last_form().form), "gemm wide stream-k w=12 kg=1 bn=%d rg=1 wgs=%d", BN, cu_count);
+        else
+            std::snprintf(last_form().form, sizeof(last_form().form), "gemm%s w=%d kg=%d bn=%d rg=%d split=%d", cfg.wide ? " wide" : "", cfg.w, cfg.kg,
+                          BN, cfg.rg, L.split);
+        e = hipLaunchKernel(fn, grid, dim3((unsigned) (64 * cfg.w)), args, lds, stream);
+    }
     if (e != hipSuccess || (L.split == 1 && !cfg.sk)) return e;
     bool yvec = a.y_s2 % 4 == 0 && a.y_s3 % 4 == 0;
     for (int j = 0; j < nmat; ++j) yvec = yvec && (reinterpret_cast<uintptr_t>(mats[j].y) & 15) == 0 && mats[j].M % 4 == 0 && mats[j].y_s1 % 4 == 0;
