@@ -472,6 +472,12 @@ __device__ __forceinline__ f32x16 mma32(const f16x8 & a, const f16x8 & b, const 
     else return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
+// Grouped MUL_MAT_ID's routing tables: a token tile's first pair, expert and pair count (0: past
+// the call's tiles) in 8 bytes; the pairs (at most 65535) in 2 bytes each.
+__device__ __forceinline__ uint2 ga_tile(int expert, int first, int count) {
+    return make_uint2((uint32_t) first, (uint32_t) expert << 8 | (uint32_t) count);
+}
+
 struct MmArgs {
     MatArgs a;
     const uint16_t * xb; // f16 activations [slices][N][K], each row scaled (k_x_to_f16)
@@ -483,13 +489,12 @@ struct MmArgs {
     int64_t stages;      // stages of K (BK elements each)
     int split;           // work-groups along K per tile
     int sk_g;            // stream-K (k_gemm_w<.., SK>): the work-groups sharing the tiles' stages
-    // grouped MUL_MAT_ID (GA kernels): pair p = t * n_used + slot; pairs[] grouped by expert,
-    // expert e's pairs at e_off[e] .. e_off[e + 1] and token tiles at t_start[e] .. t_start[e + 1];
+    // grouped MUL_MAT_ID (GA kernels): pair p = t * n_used + slot; the pairs grouped by expert in
+    // pairs[]; token tile i as ga_tile packs it;
     // x row of a pair: t * x_cols + (x_cols > 1 ? slot : 0); y of a pair: a.y + slot * a.y_s1 + t * a.y_s2
-    const int32_t * pairs;
-    const int32_t * e_off;
-    const int32_t * t_start;
-    int32_t n_used, n_exp, x_cols;
+    const uint16_t * pairs;
+    const uint2 * ga_tiles;
+    int32_t n_used, x_cols;
     // nmat weights sharing x (prefill MUL_MAT_MULTI; one slice when nmat > 1): matrix j owns row
     // tiles mt[j] .. mt[j + 1] and columns mo[j] .. mo[j + 1] of the split-K partials (entries
     // from nmat on repeat the totals); nmat = 1 mirrors `a`. packed: the row tiles run over all
@@ -654,22 +659,26 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     int64_t * ga_y = reinterpret_cast<int64_t *>(ga_rows + BN);               // GA: its y element offset
     int32_t ga_cnt = BN;                                                      // GA: the tile's pairs
     bool half_tile = false;                                                   // GA: ga_cnt <= 32 (wave-uniform)
+    F f[RG];
+    RawSet ra{};
+    auto init_f = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < RG; ++i) f[i].init(M, nb, RowAddr(M, m0 + 32 * i + j), h);
+    };
     if constexpr (GA) {
-        // the expert owning token tile tn: the last e with t_start[e] <= tn (an empty expert
-        // shares its start with the next one)
-        if (tn >= L.t_start[L.n_exp]) return; // past this call's tiles (the whole work-group)
-        int lo = 0, hi = L.n_exp - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (L.t_start[mid] <= tn) lo = mid;
-            else hi = mid - 1;
-        }
-        const int32_t pb = L.e_off[lo] + (int32_t) (tn - L.t_start[lo]) * BN;
-        ga_cnt = min(BN, L.e_off[lo + 1] - pb);
+        // (one entry per tile from the routing: a search over the experts' starts here was a chain of
+        // dependent loads ahead of the tile's first weights)
+        const uint2 gt = L.ga_tiles[tn];
+        ga_cnt = (int32_t) (gt.y & 0xff);
+        if (ga_cnt == 0) return; // past this call's tiles (the whole work-group)
         half_tile = ga_cnt <= 32;
-        w = L.a.w + (uint64_t) lo * L.a.w_s2;
+        w = L.a.w + (uint64_t) (gt.y >> 8) * L.a.w_s2;
+        // (the first weights' round trip beside those of the pairs and of their x rows)
+        init_f();
+#pragma unroll
+        for (int i = 0; i < RG; ++i) ra.r[i] = f[i].load(w, 0);
         if (tid < BN) {
-            const int32_t pr = L.pairs[pb + min(tid, ga_cnt - 1)]; // tokens past the count repeat the last pair
+            const int32_t pr = L.pairs[gt.x + min(tid, ga_cnt - 1)]; // tokens past the count repeat the last pair
             const int32_t t = pr / L.n_used, slot = pr - t * L.n_used;
             ga_rows[tid] = t * L.x_cols + (L.x_cols > 1 ? slot : 0);
             ga_y[tid] = (int64_t) slot * L.a.y_s1 + (int64_t) t * L.a.y_s2;
@@ -686,14 +695,12 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     const int64_t groups = (L.stages + 3) / 4;
     // (stage indices in 32 bits: K < 2^31 elements, and scalar 32-bit compares)
     const int gsz = (int) (4 * ((groups + KG - 1) / KG));
-    const int s0 = (int) (KG > 1 ? kg * gsz : 4 * (groups * split / L.split));
-    const int s1 = (int) (KG > 1 ? min<int64_t>(s0 + gsz, L.stages) : min(4 * (groups * (split + 1) / L.split), L.stages));
+    const int s0 = (int) (KG > 1 ? kg * gsz : GA ? 0 : 4 * (groups * split / L.split));
+    const int s1 = (int) (KG > 1 ? min<int64_t>(s0 + gsz, L.stages) : GA ? L.stages : min(4 * (groups * (split + 1) / L.split), L.stages));
     const int send = KG > 1 ? s0 + gsz : s1;                      // the loop's end (KG > 1: the same count for all)
     const int lim = s1 > s0 ? s1 - 1 : (int) L.stages - 1;       // the last stage a load may read
 
-    F f[RG];
-#pragma unroll
-    for (int i = 0; i < RG; ++i) f[i].init(M, nb, RowAddr(M, m0 + 32 * i + j), h);
+    if constexpr (!GA) init_f();
     const uint16_t * xb = L.xb + (uint64_t) sl * N * K;
     XTile<BN, RW, GA> xt;
     if constexpr (GA) xt.init_rows(K, ga_rows, tid - kg * 64 * RW);
@@ -850,11 +857,13 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
         if (s + 1 < s1) xn.store(lds_x + ((D + 1) & 1) * (BN * BK));
         __syncthreads();
     };
-    RawSet ra{}, rb{};
+    RawSet rb{};
     XTile<BN, RW, GA> xt2 = xt;
     // every split has at least one stage (the host keeps split <= stages)
+    if constexpr (!GA) {
 #pragma unroll
-    for (int i = 0; i < RG; ++i) ra.r[i] = f[i].load(w, min(s0, lim));
+        for (int i = 0; i < RG; ++i) ra.r[i] = f[i].load(w, min(s0, lim));
+    }
     xt.load(xb, min(s0, lim) * BK, (int) K);
     if constexpr (XD == 2) xt2.load(xb, min(s0 + 1, lim) * BK, (int) K);
     xt.store(lds_x);
@@ -1065,22 +1074,21 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
     int64_t * ga_y = reinterpret_cast<int64_t *>(ga_rows + BN);           // its y element offset
     int32_t ga_cnt = BN;                                                  // the tile's pairs
     bool half_tile = false; // at most 32 pairs: the second token fragment is padding (wave-uniform)
+    F f;
+    Raw ra{};
     if constexpr (GA) {
-        // the expert owning token tile tn: the last e with t_start[e] <= tn (an empty expert
-        // shares its start with the next one)
-        if (tn >= L.t_start[L.n_exp]) return; // past this call's tiles (the whole work-group)
-        int lo = 0, hi = L.n_exp - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (L.t_start[mid] <= tn) lo = mid;
-            else hi = mid - 1;
-        }
-        const int32_t pb = L.e_off[lo] + (int32_t) (tn - L.t_start[lo]) * BN;
-        ga_cnt = min(BN, L.e_off[lo + 1] - pb);
+        // (one entry per tile from the routing: a search over the experts' starts here was a chain of
+        // dependent loads ahead of the tile's first weights)
+        const uint2 gt = L.ga_tiles[tn];
+        ga_cnt = (int32_t) (gt.y & 0xff);
+        if (ga_cnt == 0) return; // past this call's tiles (the whole work-group)
         half_tile = ga_cnt <= 32;
-        w = L.a.w + (uint64_t) lo * L.a.w_s2;
+        w = L.a.w + (uint64_t) (gt.y >> 8) * L.a.w_s2;
+        // (the first weights' round trip beside those of the pairs and of their x rows)
+        f.init(M, nb, RowAddr(M, m0 + j), h);
+        ra = f.load(w, 0);
         if (threadIdx.x < BN) {
-            const int32_t pr = L.pairs[pb + min((int) threadIdx.x, ga_cnt - 1)]; // tokens past the count repeat the last pair
+            const int32_t pr = L.pairs[gt.x + min((int) threadIdx.x, ga_cnt - 1)]; // tokens past the count repeat the last pair
             const int32_t t = pr / L.n_used, slot = pr - t * L.n_used;
             ga_rows[threadIdx.x] = t * L.x_cols + (L.x_cols > 1 ? slot : 0);
             ga_y[threadIdx.x] = (int64_t) slot * L.a.y_s1 + (int64_t) t * L.a.y_s2;
@@ -1099,8 +1107,7 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
     const int send = KG > 1 ? s0 + gsz : s1;
     const int lim = s1 - 1;
 
-    F f;
-    f.init(M, nb, RowAddr(M, m0 + j), h);
+    if constexpr (!GA) f.init(M, nb, RowAddr(M, m0 + j), h);
     const uint16_t * xb = L.xb + (uint64_t) sl * N * K;
     XDma<RW, BN> xt;
     if constexpr (GA) xt.init_rows(ga_rows, K, wave, lane);
@@ -1116,8 +1123,9 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
 
     // one stage: the weights of stage s + 1 into nw and its x tile into the other LDS buffer
     // (read by every wave before the last barrier) while the MFMAs run over buffer s % 2
-    auto stage = [&](auto dtag, int s, const Raw & cw, Raw & nw) __attribute__((always_inline)) {
-        constexpr int D = decltype(dtag)::value;
+    // (NQ: the tile's token fragments that hold tokens)
+    auto stage = [&](auto qtag, auto dtag, int s, const Raw & cw, Raw & nw) __attribute__((always_inline)) {
+        constexpr int D = decltype(dtag)::value, NQ = decltype(qtag)::value;
         const int sn = min(s + 1, lim);
         if constexpr ((DT == Q4_K || DT == Q6_K) && (D & 1) == 0) nw = f.load_half2(w, sn, cw);
         else nw = f.load(w, sn);
@@ -1128,9 +1136,9 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
             return;
         }
         const typename F::Sc sc = f.prep(cw, (s & ~3) | D);
-        f16x8 a[NF];
+        f16x8 a[NQ];
 #pragma unroll
-        for (int q = 0; q < NF; ++q) a[q] = *reinterpret_cast<const f16x8 *>(X + q * 32 * XR + 8 * F::chunk(h, 0));
+        for (int q = 0; q < NQ; ++q) a[q] = *reinterpret_cast<const f16x8 *>(X + q * 32 * XR + 8 * F::chunk(h, 0));
         f16x8 b = F::bop(cw, sc, 0);
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
@@ -1143,19 +1151,20 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
             f16x8 bn;
             if (t < 7) bn = F::bop(cw, sc, t + 1);
 #pragma unroll
-            for (int q = 0; q < NF; ++q) {
-                if (!(GA && q > 0 && half_tile)) acc[q] = mma32<DT>(a[q], b, acc[q]);
+            for (int q = 0; q < NQ; ++q) {
+                acc[q] = mma32<DT>(a[q], b, acc[q]);
                 if (t < 7) a[q] = *reinterpret_cast<const f16x8 *>(X + q * 32 * XR + 8 * F::chunk(h, t + 1));
             }
             if (t < 7) b = bn;
         }
         __syncthreads(); // (waits for this wave's loads: the next x tile is in LDS)
     };
-    Raw ra{}, rb{};
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
     using I3 = std::integral_constant<int, 3>;
+    auto run = [&](auto qtag) __attribute__((always_inline)) {
+    Raw rb{};
     int s = s0;
     if constexpr (SK) {
         // a piece starts at an even stage: stages 2 and 3 of a group of 4 run first when it
@@ -1165,28 +1174,35 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
         xt.load(xb, s0 * BK, lds_x);
         __syncthreads();
         if (s0 & 2) {
-            stage(I2{}, s, ra, rb);
-            if (s + 1 < s1) stage(I3{}, s + 1, rb, ra);
+            stage(qtag, I2{}, s, ra, rb);
+            if (s + 1 < s1) stage(qtag, I3{}, s + 1, rb, ra);
             s += 2;
         }
     } else {
-        ra = f.load(w, min(s0, lim));
+        if constexpr (!GA) ra = f.load(w, min(s0, lim));
         xt.load(xb, min(s0, lim) * BK, lds_x);
         __syncthreads();
     }
     for (; s + 3 < send; s += 4) {
-        stage(I0{}, s, ra, rb);
-        stage(I1{}, s + 1, rb, ra);
-        stage(I2{}, s + 2, ra, rb);
-        stage(I3{}, s + 3, rb, ra);
+        stage(qtag, I0{}, s, ra, rb);
+        stage(qtag, I1{}, s + 1, rb, ra);
+        stage(qtag, I2{}, s + 2, ra, rb);
+        stage(qtag, I3{}, s + 3, rb, ra);
     }
     if (s < send) { // (KG = 2: send - s0 is a multiple of 4, no tail)
-        stage(I0{}, s, ra, rb);
+        stage(qtag, I0{}, s, ra, rb);
         if (s + 1 < s1) {
-            stage(I1{}, s + 1, rb, ra);
-            if (s + 2 < s1) stage(I2{}, s + 2, ra, rb);
+            stage(qtag, I1{}, s + 1, rb, ra);
+            if (s + 2 < s1) stage(qtag, I2{}, s + 2, ra, rb);
         }
     }
+    };
+    // (GA: a tile of at most 32 pairs runs a loop of its own without the second token fragment's
+    // MFMAs; a branch around each of them cut every k-step into basic blocks that the compiler
+    // cannot schedule across: with the tile table and the earlier weights, gate, up and down of 128
+    // Q4_K experts of 768 x 2048, 8 of them per token, 512 tokens, 157 -> 150 us)
+    if (GA && half_tile) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, NF>{});
     // acc[q][v], lane (j, h): token n0 + 32q + 8 (v / 4) + 4h + v % 4, weight row m0 + j
     auto store_out = [&](auto qb, auto qc) __attribute__((always_inline)) {
         constexpr int QB = decltype(qb)::value, QC = decltype(qc)::value;
@@ -1663,20 +1679,21 @@ __global__ __launch_bounds__(256) void k_x_to_f16(MatArgs a, uint16_t * xb, floa
     x_row_to_f16<VEC, Q4K, BF, FRAG, PLAIN>(a, xb, xs, xsum, xsum_row, blockIdx.x, threadIdx.x, wmax, true);
 }
 
-// MUL_MAT_ID routing (E <= 1024 experts, P < 2^24 pairs), by one 1024-thread work-group: the
-// pairs p = t * n_used + slot grouped by expert (ids clamped to [0, E)); e_off[e] / t_start[e] =
-// the first pair / token tile (bn pairs) of expert e, [E] = the totals. Counts with LDS atomics,
-// exclusive scans of the counts and of the tile counts (one expert per thread, wave scans), then
-// each pair placed at its expert's cursor (its id read again: it is in the L2 by then). The order
+// MUL_MAT_ID routing (E <= 1024 experts, P < 2^16 pairs), by one 1024-thread work-group: the
+// pairs p = t * n_used + slot grouped by expert (ids clamped to [0, E)), and per token tile (bn
+// pairs) its expert, first pair and count, 0 past the last tile. Counts with LDS atomics,
+// exclusive scans of the counts and of the tile counts (one expert per thread, wave scans), each
+// expert's tiles written by its thread, then each pair placed at its expert's cursor (its id read
+// again: it is in the L2 by then). The order
 // of the pairs inside an expert follows the LDS atomics; no output depends on it (each is one
 // pair's own sum over K).
 struct RouteArgs {
     const int32_t * ids;
     int64_t s0, s1;
     int nu, T, E, bn;
-    int32_t * e_off;
-    int32_t * t_start;
-    int32_t * pairs;
+    uint16_t * pairs;
+    uint2 * tiles; // n_tiles entries
+    int n_tiles;
 };
 
 __device__ __forceinline__ void moe_route(const RouteArgs & r) {
@@ -1712,17 +1729,13 @@ __device__ __forceinline__ void moe_route(const RouteArgs & r) {
         ea += wsum[0][w2];
         eb += wsum[1][w2];
     }
-    if (tid < r.E) {
-        r.e_off[tid] = ea;
-        r.t_start[tid] = eb;
-        cur[tid] = ea;
-    }
-    if (tid == r.E - 1) {
-        r.e_off[r.E] = ea + c;
-        r.t_start[r.E] = eb + tl;
-    }
+    cur[tid] = ea;
+    int total = 0; // token tiles of all experts
+    for (int w2 = 0; w2 < 16; ++w2) total += wsum[1][w2];
+    for (int k = 0; k < tl; ++k) r.tiles[eb + k] = ga_tile(tid, ea + k * r.bn, min(r.bn, c - k * r.bn));
+    for (int i = total + tid; i < r.n_tiles; i += 1024) r.tiles[i] = make_uint2(0, 0);
     __syncthreads();
-    for (int p = tid; p < P; p += 1024) r.pairs[atomicAdd(&cur[expert(p)], 1)] = p;
+    for (int p = tid; p < P; p += 1024) r.pairs[atomicAdd(&cur[expert(p)], 1)] = (uint16_t) p;
 }
 
 // the grouped MUL_MAT_ID's first launch: work-group 0 routes the pairs while the others convert
@@ -2419,6 +2432,11 @@ int ga_bn(const IdArgs & id) {
     return id.n_used * id.n_tok >= 16 * id.n_exp ? 64 : 32;
 }
 
+// at least the token tiles the routing makes
+int64_t ga_tiles(const IdArgs & id) {
+    return (id.n_used * id.n_tok + ga_bn(id) - 1) / ga_bn(id) + id.n_exp;
+}
+
 // the pre-pass's view of MUL_MAT_ID's x: rows t * x_cols + c at x + c * x_s1 + t * x_s2
 MatArgs ga_xargs(const MatArgs & a, const IdArgs & id) {
     MatArgs px = a;
@@ -2448,7 +2466,7 @@ int ga_waves(const MatArgs & a, const IdArgs & id, int cu_count) {
 
 size_t mul_mat_id_scratch_bytes(const MatArgs & a, const IdArgs & id) {
     const MatArgs px = ga_xargs(a, id);
-    return part_offset(px) + (size_t) (2 * (id.n_exp + 1) + id.n_used * id.n_tok) * sizeof(int32_t);
+    return part_offset(px) + (size_t) ga_tiles(id) * sizeof(uint2) + (size_t) (id.n_used * id.n_tok) * sizeof(uint16_t);
 }
 
 // the grouped path's x form: the wide GEMM (plain f16 x) or k_matmul (its single-fma Q4_K form)
@@ -2466,7 +2484,7 @@ hipError_t launch_mul_mat_id_mfma(const MatArgs & a, const IdArgs & id, uint8_t 
                                   bool x_ready) {
     const MatArgs px = ga_xargs(a, id);
     const int64_t rows = px.N * id.n_tok;
-    if (id.n_exp < 1 || id.n_exp > 1024 || rows * a.K >= ((int64_t) 1 << 31) || id.n_used * id.n_tok >= ((int64_t) 1 << 24)) return hipErrorInvalidValue;
+    if (id.n_exp < 1 || id.n_exp > 1024 || rows * a.K >= ((int64_t) 1 << 31) || id.n_used * id.n_tok >= ((int64_t) 1 << 16)) return hipErrorInvalidValue;
     uint16_t * xb = reinterpret_cast<uint16_t *>(scratch);
     float * xs = reinterpret_cast<float *>(scratch + xs_offset(px));
     uint16_t * xsum = reinterpret_cast<uint16_t *>(scratch + xsum_offset(px));
@@ -2477,10 +2495,9 @@ hipError_t launch_mul_mat_id_mfma(const MatArgs & a, const IdArgs & id, uint8_t 
     // 384-row x 64-token tiles on the wide GEMM where K is a whole number of stages (x tiles
     // straight into LDS, the exact Q4_K form from plain x)
     const bool wide = ga_wide(a, id, cu_count);
-    int32_t * e_off = reinterpret_cast<int32_t *>(scratch + part_offset(px));
-    int32_t * t_start = e_off + id.n_exp + 1;
-    int32_t * pairs = t_start + id.n_exp + 1;
-    const RouteArgs ra{id.ids, id.s0, id.s1, (int) id.n_used, (int) id.n_tok, (int) id.n_exp, bn, e_off, t_start, pairs};
+    uint2 * tiles = reinterpret_cast<uint2 *>(scratch + part_offset(px)); // (256-byte aligned)
+    uint16_t * pairs = reinterpret_cast<uint16_t *>(tiles + ga_tiles(id));
+    const RouteArgs ra{id.ids, id.s0, id.s1, (int) id.n_used, (int) id.n_tok, (int) id.n_exp, bn, pairs, tiles, (int) ga_tiles(id)};
     // (work-group 0 routes the pairs, the others convert the x rows)
     const dim3 xrg((unsigned) ((rows + 3) / 4 + 1));
     if (x_ready) {
@@ -2514,12 +2531,10 @@ hipError_t launch_mul_mat_id_mfma(const MatArgs & a, const IdArgs & id, uint8_t 
     L.stages = (a.K + BK - 1) / BK;
     L.tiles_m = (a.M + 32 * waves - 1) / (32 * waves);
     L.mt[1] = L.mt[2] = L.mt[3] = L.tiles_m;
-    L.tiles_n = (id.n_used * id.n_tok + bn - 1) / bn + id.n_exp; // at least the tiles the routing makes
+    L.tiles_n = ga_tiles(id);
     L.pairs = pairs;
-    L.e_off = e_off;
-    L.t_start = t_start;
+    L.ga_tiles = tiles;
     L.n_used = (int32_t) id.n_used;
-    L.n_exp = (int32_t) id.n_exp;
     L.x_cols = (int32_t) px.N;
     const size_t lds = (size_t) 2 * bn * (wide ? XR : BK) * sizeof(uint16_t) + (size_t) bn * (sizeof(int32_t) + sizeof(int64_t));
     void * fn = nullptr;

@@ -1,0 +1,52 @@
+"""The token tiles of the grouped MUL_MAT_ID: pair counts at the edges of a tile and of its half,
+experts without pairs, and the most pairs (65535) in about as many tiles as the routing has
+threads. Tolerance as
+for every prefill matmul (f16 activations): NMSE 5e-5."""
+import numpy as np
+import pytest
+
+import oracle as O
+import scrapgpulibrary_amd as sg
+from tests.test_gpu_mul_mat_id import check_grouped, run_mul_mat_id
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [sg.Q4_K, sg.Q6_K, sg.Q8_0], ids=lambda d: sg.NAMES[d])
+@pytest.mark.parametrize("form", ["wide", "tiled"])
+def test_pair_counts_at_tile_edges(hip, dtype, form):
+    """One slot per token: expert e gets counts[e] pairs; with bn = 64 a tile of at most 32 runs
+    without its second fragment."""
+    dev, st = hip
+    counts = [0, 1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 0]
+    K, M = 512, 384
+    if form == "wide":  # 384-row tiles need half as many experts as CUs
+        counts = counts + [0, 40] * 64
+    E = len(counts)
+    ids = np.repeat(np.arange(E), counts).astype(np.int32)
+    ids = np.random.default_rng(91).permutation(ids).reshape(-1, 1)
+    T = len(ids)
+    w = O.quantize(dtype, O.normal(K * M * E, 92, 0.0, 0.02))
+    x = O.normal(T * K, 93).reshape(T, 1, K)
+    y = run_mul_mat_id(dev, st, dtype, w, K, M, E, x, ids)
+    if dev.info().compute_units == 256:
+        assert sg.last_launch()[0] == ("grouped wide w=12 bn=64" if form == "wide" else "grouped w=4 bn=64"), sg.last_launch()
+    check_grouped(y, O.mul_mat_id(dtype, w, K, M, E, x, ids))
+
+
+def test_many_tiles_and_pairs(hip):
+    """65535 pairs, the most a call may have, over 3 experts (1026 or 1027 token tiles)."""
+    dev, st = hip
+    K, M, E, T, nu = 256, 64, 3, 21845, 3
+    rng = np.random.default_rng(94)
+    ids = rng.integers(0, E, (T, nu)).astype(np.int32)
+    w = O.quantize(sg.Q4_0, O.normal(K * M * E, 95, 0.0, 0.02))
+    x = O.normal(T * K, 96).reshape(T, 1, K)
+    y = run_mul_mat_id(dev, st, sg.Q4_0, w, K, M, E, x, ids)
+    deq = O.dequantize(sg.Q4_0, w, K * M * E).reshape(E, M, K).astype(np.float64)
+    xd = x[:, 0].astype(np.float64)
+    per = np.stack([xd @ deq[e].T for e in range(E)], 1)  # every token against every expert
+    ref = np.take_along_axis(per, ids[:, :, None], 1)
+    d = ((y - ref) ** 2).sum(2) / (ref ** 2).sum(2)
+    assert d.max() <= 20 * 5e-5, (d.max(), int(d.argmax()))
+    assert ((y - ref) ** 2).sum() <= 5e-5 * (ref ** 2).sum()
