@@ -478,6 +478,38 @@ __device__ __forceinline__ uint2 ga_tile(int expert, int first, int count) {
     return make_uint2((uint32_t) first, (uint32_t) expert << 8 | (uint32_t) count);
 }
 
+// Index arithmetic ahead of a kernel's first load. A 64-bit division is tens of dependent
+// instructions (a call over few tokens has up to ten of them before it asks for its first weights),
+// so a quotient that the usual call knows, 0 or 1 for one slice and one split, is not divided for,
+// and tile numbers (the grid's x extent) are divided in 32 bits.
+struct Slice {
+    int64_t i2, i3;
+};
+__device__ __forceinline__ Slice slice_of(const MatArgs & a, int64_t sl) { // x slice sl
+    if (sl == 0) return {0, 0};
+    const int64_t i3 = sl / a.ne12;
+    return {sl - i3 * a.ne12, i3};
+}
+__device__ __forceinline__ int64_t slice_w(const MatArgs & a, const Slice & c) { // its weights' byte offset
+    int64_t o = 0;
+    if (c.i2 != 0) o += (int64_t) ((uint64_t) (c.i2 / a.r2) * a.w_s2);
+    if (c.i3 != 0) o += (int64_t) ((uint64_t) (c.i3 / a.r3) * a.w_s3);
+    return o;
+}
+__device__ __forceinline__ int64_t row_slice(int64_t row, int64_t n) { return row < n ? 0 : row / n; } // the slice of x row `row`
+// the first stage of a split (K in groups of 4 stages; split = n: K's end, or up to 3 past it)
+__device__ __forceinline__ int64_t split_start(int64_t groups, int split, int n) {
+    if (split == 0) return 0;
+    return 4 * (split == n ? groups : groups * split / n);
+}
+struct TileOf {
+    int64_t tm, tn;
+};
+__device__ __forceinline__ TileOf tile_of(int64_t tile, int64_t tiles_m) {
+    const uint32_t t = (uint32_t) tile, m = (uint32_t) tiles_m, q = t / m;
+    return {(int64_t) (t - q * m), (int64_t) q};
+}
+
 struct MmArgs {
     MatArgs a;
     const uint16_t * xb; // f16 activations [slices][N][K], each row scaled (k_x_to_f16)
@@ -639,17 +671,18 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = (tid >> 6) % RW, kg = (tid >> 6) / RW; // row wave, K group
     const int j = lane & 31, h = lane >> 5;
-    const int64_t tile = blockIdx.x / L.split;
-    const int split = (int) (blockIdx.x % L.split);
-    const int64_t tm = tile % L.tiles_m, tn = tile / L.tiles_m;
+    const uint32_t tile = L.split == 1 ? blockIdx.x : blockIdx.x / (uint32_t) L.split;
+    const int split = (int) (blockIdx.x - tile * (uint32_t) L.split);
+    const TileOf at = tile_of(tile, L.tiles_m);
+    const int64_t tm = at.tm, tn = at.tn;
     const int64_t sl = blockIdx.y;
-    const int64_t i2 = sl % L.a.ne12, i3 = sl / L.a.ne12;
+    const Slice slc = slice_of(L.a, sl);
     // the wave's matrix (several when weights share x)
     const int64_t grow = tm * BMT + 32 * RG * wave; // packed: the wave's first row over all matrices
     const int mj = L.nmat == 1 ? 0
                  : L.packed    ? min(L.nmat - 1, grow >= L.mo[1] ? (grow >= L.mo[2] ? 2 : 1) : 0)
                                : (tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0);
-    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + (uint64_t) (i2 / L.a.r2) * L.a.w_s2 + (uint64_t) (i3 / L.a.r3) * L.a.w_s3;
+    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + slice_w(L.a, slc);
     const int64_t K = L.a.K, nb = L.a.nb;
     const int64_t M = L.nmat > 1 ? L.Mm[mj] : L.a.M;
     int64_t N = L.a.N;
@@ -695,8 +728,8 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     const int64_t groups = (L.stages + 3) / 4;
     // (stage indices in 32 bits: K < 2^31 elements, and scalar 32-bit compares)
     const int gsz = (int) (4 * ((groups + KG - 1) / KG));
-    const int s0 = (int) (KG > 1 ? kg * gsz : GA ? 0 : 4 * (groups * split / L.split));
-    const int s1 = (int) (KG > 1 ? min<int64_t>(s0 + gsz, L.stages) : GA ? L.stages : min(4 * (groups * (split + 1) / L.split), L.stages));
+    const int s0 = (int) (KG > 1 ? kg * gsz : GA ? 0 : split_start(groups, split, L.split));
+    const int s1 = (int) (KG > 1 ? min<int64_t>(s0 + gsz, L.stages) : GA ? L.stages : min(split_start(groups, split + 1, L.split), L.stages));
     const int send = KG > 1 ? s0 + gsz : s1;                      // the loop's end (KG > 1: the same count for all)
     const int lim = s1 > s0 ? s1 - 1 : (int) L.stages - 1;       // the last stage a load may read
 
@@ -923,7 +956,7 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     float * y;
     int64_t ys1;
     if (L.split == 1) {
-        y = L.nmat > 1 ? L.ym[mj] : L.a.y + i2 * L.a.y_s2 + i3 * L.a.y_s3;
+        y = L.nmat > 1 ? L.ym[mj] : L.a.y + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
         ys1 = L.nmat > 1 ? L.ys1m[mj] : L.a.y_s1;
     } else {
         const int64_t mt_all = L.mo[L.nmat]; // the partials' row length: all matrices' rows
@@ -1054,14 +1087,15 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
     // k_sk_reduce adds in work-group order (g + t rises by at least one from piece to piece, so
     // the slots are distinct)
     auto piece = [&](const int64_t tile, const int split, const int p0, const int p1, const int64_t slot) __attribute__((always_inline)) {
-    const int64_t tm = tile % L.tiles_m, tn = tile / L.tiles_m;
+    const TileOf at = tile_of(tile, L.tiles_m);
+    const int64_t tm = at.tm, tn = at.tn;
     const int64_t sl = blockIdx.y;
-    const int64_t i2 = sl % L.a.ne12, i3 = sl / L.a.ne12;
+    const Slice slc = slice_of(L.a, sl);
     const int64_t grow = tm * BMT + 32 * wave;
     const int mj = L.nmat == 1 ? 0
                  : L.packed    ? min(L.nmat - 1, grow >= L.mo[1] ? (grow >= L.mo[2] ? 2 : 1) : 0)
                                : (tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0);
-    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + (uint64_t) (i2 / L.a.r2) * L.a.w_s2 + (uint64_t) (i3 / L.a.r3) * L.a.w_s3;
+    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + slice_w(L.a, slc);
     const int64_t K = L.a.K, nb = L.a.nb;
     int64_t N = L.a.N;
     const int64_t M = L.nmat > 1 ? L.Mm[mj] : L.a.M;
@@ -1102,8 +1136,8 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
     // are inactive: their loads repeat a valid stage, their k-steps are skipped), as in k_matmul
     const int64_t groups = (L.stages + 3) / 4;
     const int gsz = (int) (4 * ((groups + KG - 1) / KG));
-    const int s0 = SK ? p0 : (int) (KG > 1 ? kg * gsz : 4 * (groups * split / L.split));
-    const int s1 = SK ? p1 : (int) (KG > 1 ? min<int64_t>(s0 + gsz, L.stages) : min(4 * (groups * (split + 1) / L.split), L.stages));
+    const int s0 = SK ? p0 : (int) (KG > 1 ? kg * gsz : split_start(groups, split, L.split));
+    const int s1 = SK ? p1 : (int) (KG > 1 ? min<int64_t>(s0 + gsz, L.stages) : min(split_start(groups, split + 1, L.split), L.stages));
     const int send = KG > 1 ? s0 + gsz : s1;
     const int lim = s1 - 1;
 
@@ -1230,7 +1264,7 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
             y = L.part + (uint64_t) slot * (BN * BMT) - n0 * BMT + 32 * wave + j - m;
             ys1 = BMT;
         } else if (L.split == 1) {
-            y = L.nmat > 1 ? L.ym[mj] : L.a.y + i2 * L.a.y_s2 + i3 * L.a.y_s3;
+            y = L.nmat > 1 ? L.ym[mj] : L.a.y + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
             ys1 = L.nmat > 1 ? L.ys1m[mj] : L.a.y_s1;
         } else {
             const int64_t mt_all = L.mo[L.nmat];
@@ -1318,7 +1352,8 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
             lo = (t + 1) * S;
         }
     } else {
-        piece(blockIdx.x / L.split, (int) (blockIdx.x % L.split), 0, 0, -1);
+        const uint32_t tile = L.split == 1 ? blockIdx.x : blockIdx.x / (uint32_t) L.split;
+        piece(tile, (int) (blockIdx.x - tile * (uint32_t) L.split), 0, 0, -1);
     }
 }
 
@@ -1350,9 +1385,9 @@ __global__ __launch_bounds__(64 * KW * RW) void k_gemm_n(MmArgs L) {
     // the wave's R32 group (past the last one: the last one again, not stored)
     const int64_t tm = min<int64_t>((int64_t) blockIdx.x * RW + rw, L.tiles_m - 1), sl = blockIdx.y;
     const bool live = (int64_t) blockIdx.x * RW + rw < L.tiles_m;
-    const int64_t i2 = sl % L.a.ne12, i3 = sl / L.a.ne12;
+    const Slice slc = slice_of(L.a, sl);
     const int mj = L.nmat == 1 ? 0 : (tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0);
-    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + (uint64_t) (i2 / L.a.r2) * L.a.w_s2 + (uint64_t) (i3 / L.a.r3) * L.a.w_s3;
+    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + slice_w(L.a, slc);
     const int64_t nb = L.a.nb, N = L.a.N;
     const int64_t M = L.nmat > 1 ? L.Mm[mj] : L.a.M;
     const int64_t m0 = (tm - L.mt[mj]) * 32;
@@ -1442,7 +1477,7 @@ __global__ __launch_bounds__(64 * KW * RW) void k_gemm_n(MmArgs L) {
         if (r > 1) __syncthreads();
     }
     if (kw != 0 || !live) return;
-    float * y = L.nmat > 1 ? L.ym[mj] : L.a.y + i2 * L.a.y_s2 + i3 * L.a.y_s3;
+    float * y = L.nmat > 1 ? L.ym[mj] : L.a.y + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
     const int64_t ys1 = L.nmat > 1 ? L.ys1m[mj] : L.a.y_s1;
     const float * xs = L.xs + (uint64_t) sl * N;
     const int64_t m = m0 + j;
@@ -1461,13 +1496,13 @@ __global__ __launch_bounds__(64 * KW * RW) void k_gemm_n(MmArgs L) {
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_split_reduce(MmArgs L) {
     const int64_t N = L.a.N, Mt = L.mo[L.nmat];
-    const int64_t row = blockIdx.x, sl = row / N, n = row - sl * N;
-    const int64_t i2 = sl % L.a.ne12, i3 = sl / L.a.ne12;
+    const int64_t row = blockIdx.x, sl = row_slice(row, N), n = row - sl * N;
+    const Slice slc = slice_of(L.a, sl);
     const uint64_t plane = (uint64_t) L.a.ne12 * L.a.ne13 * N * Mt;
     const float * p = L.part + row * Mt;
     auto out = [&](int64_t c) -> float * { // y element of column c
         const int j = c >= L.mo[1] ? (c >= L.mo[2] ? 2 : 1) : 0;
-        float * y = L.nmat > 1 ? L.ym[j] + n * L.ys1m[j] : L.a.y + i2 * L.a.y_s2 + i3 * L.a.y_s3 + n * L.a.y_s1;
+        float * y = L.nmat > 1 ? L.ym[j] + n * L.ys1m[j] : L.a.y + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3 + n * L.a.y_s1;
         return y + (c - L.mo[j]);
     };
     const int64_t m = ((int64_t) blockIdx.y * 256 + threadIdx.x) * 4;
@@ -1567,9 +1602,9 @@ template <bool VEC, bool Q4K, bool BF, bool FRAG, bool PLAIN>
 __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, float * xs, uint16_t * xsum, int64_t xsum_row, int64_t row,
                                              int tid, float * wmax, bool live) {
     constexpr int kCached = 6; // K <= 12288 is read once
-    const int64_t sl = row / a.N, n = row - sl * a.N;
-    const int64_t i2 = sl % a.ne12, i3 = sl / a.ne12;
-    const float * xp = a.x + i2 * a.x_s2 + i3 * a.x_s3 + n * a.x_s1;
+    const int64_t sl = row_slice(row, a.N), n = row - sl * a.N;
+    const Slice slc = slice_of(a, sl);
+    const float * xp = a.x + slc.i2 * a.x_s2 + slc.i3 * a.x_s3 + n * a.x_s1;
     uint16_t * op = xb + row * a.K;
     if constexpr (FRAG)
         op = xb + ((sl * ((a.N + 31) / 32) + n / 32) * (a.K / BK) * kChunks * 32 + n % 32) * 8;
