@@ -1596,12 +1596,13 @@ __global__ __launch_bounds__(256) void k_sk_reduce(MmArgs L) {
 // chunk c (8 elements) of stage s of token n at ((n / 32 * stages + s) * 16 + c) * 32 + n % 32 in
 // units of 16 bytes (per slice, tokens padded to a multiple of 32): the 32 tokens of one chunk
 // are 512 contiguous bytes.
-// (tid: the thread's index among the row's 256, wmax: 4 floats of LDS for the row's waves; a
-// thread group with live = false takes part in the barrier only)
-template <bool VEC, bool Q4K, bool BF, bool FRAG, bool PLAIN>
+// (tid: the thread's index among the row's TPR = 256, wmax: 4 floats of LDS for the row's waves; a
+// thread group with live = false takes part in the barrier only. TPR = 64: one wave, no barrier)
+template <bool VEC, bool Q4K, bool BF, bool FRAG, bool PLAIN, int TPR = 256>
 __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, float * xs, uint16_t * xsum, int64_t xsum_row, int64_t row,
                                              int tid, float * wmax, bool live) {
-    constexpr int kCached = 6; // K <= 12288 is read once
+    constexpr int kCached = 6; // K <= 12288 is read once (TPR = 64: 3072)
+    constexpr int STEP = 8 * TPR;
     const int64_t sl = row_slice(row, a.N), n = row - sl * a.N;
     const Slice slc = slice_of(a, sl);
     const float * xp = a.x + slc.i2 * a.x_s2 + slc.i3 * a.x_s3 + n * a.x_s1;
@@ -1665,14 +1666,14 @@ __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, f
     float mx = 0.0f;
 #pragma unroll
     for (int c = 0; c < kCached; ++c) {
-        const int64_t k = k0 + (int64_t) c * 2048;
+        const int64_t k = k0 + (int64_t) c * STEP;
         if (k < a.K) {
             load8(k, cache[c]);
 #pragma unroll
             for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(cache[c][e]));
         }
     }
-    for (int64_t k = k0 + (int64_t) kCached * 2048; k < a.K; k += 2048) {
+    for (int64_t k = k0 + (int64_t) kCached * STEP; k < a.K; k += STEP) {
         float v[8];
         load8(k, v);
 #pragma unroll
@@ -1680,9 +1681,11 @@ __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, f
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if ((tid & 63) == 0) wmax[tid >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    if constexpr (TPR == 256) {
+        if ((tid & 63) == 0) wmax[tid >> 6] = mx;
+        __syncthreads();
+        mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    }
     int e2 = 0;
     if (mx > 0.0f && mx <= 3.4e38f) {
         int ex;
@@ -1692,16 +1695,16 @@ __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, f
     if (tid == 0 && live) xs[row] = ldexpf(1.0f, -e2);
 #pragma unroll
     for (int c = 0; c < kCached; ++c) {
-        const int64_t k = k0 + (int64_t) c * 2048;
+        const int64_t k = k0 + (int64_t) c * STEP;
         if (k < a.K) store8(k, cache[c], e2);
     }
-    for (int64_t k = k0 + (int64_t) kCached * 2048; k < a.K; k += 2048) {
+    for (int64_t k = k0 + (int64_t) kCached * STEP; k < a.K; k += STEP) {
         float v[8];
         load8(k, v);
         store8(k, v, e2);
     }
     if constexpr (Q4K) {
-        for (int64_t jb = a.K / 32 + tid; live && jb < xsum_row; jb += 256) {
+        for (int64_t jb = a.K / 32 + tid; live && jb < xsum_row; jb += TPR) {
             const int64_t jj = jb & 15;
             xsum[row * xsum_row + (jb >> 4) * 16 + 8 * ((jj >> 1) & 1) + 2 * (jj >> 2) + (jj & 1)] = 0;
         }
@@ -1774,9 +1777,10 @@ __device__ __forceinline__ void moe_route(const RouteArgs & r) {
 }
 
 // the grouped MUL_MAT_ID's first launch: work-group 0 routes the pairs while the others convert
-// the x rows, 4 per work-group (k_x_to_f16's work, rows 4 (blockIdx.x - 1) + threadIdx.x / 256):
-// the routing's round trips run beside the conversion instead of in a launch of their own
-template <bool VEC, bool Q4K>
+// the x rows, 1024 / TPR per work-group (k_x_to_f16's work): the routing's round trips run beside
+// the conversion instead of in a launch of their own. TPR = 64 where 256 threads of 8 elements each
+// would be partly idle (4096 rows of 768: 12.8 -> 9.5 us)
+template <bool VEC, bool Q4K, int TPR>
 __global__ __launch_bounds__(1024) void k_x_route(MatArgs a, uint16_t * xb, float * xs, uint16_t * xsum, int64_t xsum_row, int64_t rows,
                                                   RouteArgs r) {
     if (blockIdx.x == 0) {
@@ -1784,10 +1788,10 @@ __global__ __launch_bounds__(1024) void k_x_route(MatArgs a, uint16_t * xb, floa
         return;
     }
     __shared__ float wmax[16];
-    const int q = threadIdx.x >> 8;
-    const int64_t row = 4 * ((int64_t) blockIdx.x - 1) + q;
+    const int q = threadIdx.x / TPR;
+    const int64_t row = 1024 / TPR * ((int64_t) blockIdx.x - 1) + q;
     const bool live = row < rows;
-    x_row_to_f16<VEC, Q4K, false, false, false>(a, xb, xs, xsum, xsum_row, live ? row : 0, threadIdx.x & 255, wmax + 4 * q, live);
+    x_row_to_f16<VEC, Q4K, false, false, false, TPR>(a, xb, xs, xsum, xsum_row, live ? row : 0, threadIdx.x % TPR, TPR == 256 ? wmax + 4 * q : wmax, live);
 }
 
 int env_int(const char * name, int dflt) {
@@ -2534,19 +2538,23 @@ hipError_t launch_mul_mat_id_mfma(const MatArgs & a, const IdArgs & id, uint8_t 
     uint16_t * pairs = reinterpret_cast<uint16_t *>(tiles + ga_tiles(id));
     const RouteArgs ra{id.ids, id.s0, id.s1, (int) id.n_used, (int) id.n_tok, (int) id.n_exp, bn, pairs, tiles, (int) ga_tiles(id)};
     // (work-group 0 routes the pairs, the others convert the x rows)
-    const dim3 xrg((unsigned) ((rows + 3) / 4 + 1));
+    const bool wave_row = a.K < 2048;
+    const dim3 xrg((unsigned) (wave_row ? (rows + 15) / 16 + 1 : (rows + 3) / 4 + 1));
+    const auto convert = [&](auto k64, auto k256) {
+        hipLaunchKernelGGL(wave_row ? k64 : k256, xrg, dim3(1024), 0, stream, px, xb, xs, xsum, xsum_row, rows, ra);
+    };
     if (x_ready) {
         // x converted and the pairs routed by the previous grouped MUL_MAT_ID (mul_mat_id_same_x)
     } else if (a.dtype == Q4_K && !wide) {
         if (vec)
-            hipLaunchKernelGGL((k_x_route<true, true>), xrg, dim3(1024), 0, stream, px, xb, xs, xsum, xsum_row, rows, ra);
+            convert(k_x_route<true, true, 64>, k_x_route<true, true, 256>);
         else
-            hipLaunchKernelGGL((k_x_route<false, true>), xrg, dim3(1024), 0, stream, px, xb, xs, xsum, xsum_row, rows, ra);
+            convert(k_x_route<false, true, 64>, k_x_route<false, true, 256>);
     } else {
         if (vec)
-            hipLaunchKernelGGL((k_x_route<true, false>), xrg, dim3(1024), 0, stream, px, xb, xs, xsum, xsum_row, rows, ra);
+            convert(k_x_route<true, false, 64>, k_x_route<true, false, 256>);
         else
-            hipLaunchKernelGGL((k_x_route<false, false>), xrg, dim3(1024), 0, stream, px, xb, xs, xsum, xsum_row, rows, ra);
+            convert(k_x_route<false, false, 64>, k_x_route<false, false, 256>);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -50,3 +50,21 @@ def test_many_tiles_and_pairs(hip):
     d = ((y - ref) ** 2).sum(2) / (ref ** 2).sum(2)
     assert d.max() <= 20 * 5e-5, (d.max(), int(d.argmax()))
     assert ((y - ref) ** 2).sum() <= 5e-5 * (ref ** 2).sum()
+
+
+@pytest.mark.parametrize("dtype,K", [(sg.Q4_0, 32), (sg.Q8_0, 992), (sg.Q4_0, 2016), (sg.Q8_0, 2048), (sg.Q4_K, 256), (sg.Q4_K, 1792), (sg.Q6_K, 768)],
+                         ids=lambda v: str(v))
+def test_x_rows_by_wave_and_by_group(hip, dtype, K):
+    """The conversion of x beside the routing: a wave per row below K = 2048, 4 waves from there on;
+    21 tokens with a row per slot (63 rows: the last work-group of 16 is part empty), row magnitudes
+    over six decades (each row has a scale of its own)."""
+    dev, st = hip
+    M, E, T, nu = 96, 4, 21, 3
+    rng = np.random.default_rng(97)
+    ids = np.stack([rng.permutation(E)[:nu] for _ in range(T)]).astype(np.int32)
+    w = O.quantize(dtype, O.normal(K * M * E, 98, 0.0, 0.02))
+    x = O.normal(T * nu * K, 99).reshape(T, nu, K) * (10.0 ** rng.integers(-3, 4, (T, nu, 1))).astype(np.float32)
+    y = run_mul_mat_id(dev, st, dtype, w, K, M, E, x, ids)
+    ref = O.mul_mat_id(dtype, w, K, M, E, x, ids)
+    d = ((y.astype(np.float64) - ref) ** 2).sum(2) / (ref.astype(np.float64) ** 2).sum(2)
+    assert d.max() <= 20 * 5e-5, d.max()
