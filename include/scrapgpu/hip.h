@@ -57,7 +57,8 @@ SCRAPGPU_API scrapgpu_status scrapgpu_hip_profile_read(size_t index, const char 
  * scrapgpu_op_execute runs in a stream-K form (its 384-row tiles fewer than the CUs, or a second
  * round of them at most a quarter full, and a long K) runs
  * another GEMM form here, whose output differs in rounding (both within the prefill tolerance),
- * because stream-K's partial slots do not fit the static array. An op that needs more than 32 MiB
+ * because stream-K's partial slots do not fit the static array; likewise an F16 / BF16 prefill
+ * whose K splits' partial sums would not fit takes fewer splits. An op that needs more than 32 MiB
  * of scratch is refused with SCRAPGPU_STATUS_UNSUPPORTED and a reason (decode matvecs need at most
  * a few MiB; prefill needs about 2 * N * K bytes plus, for split-K shapes, 4 * splits * N * M bytes).
  * Every call on one GPU shares that GPU's array: calls whose work overlaps on one GPU (two
