@@ -809,7 +809,7 @@ double weight_bytes(const sgk::MatArgs & a) {
 }
 
 // enqueues 1..3 products on the stream (pointers resolved). Products that share x with one dtype,
-// K and N <= 8 run as one fused matvec launch; anything else as one launch per product.
+// K, row stride and N <= 8 run as one fused matvec launch; anything else as one launch per product.
 // MUL_MAT_ID takes the grouped MFMA path for more than 8 tokens once the experts average 4 pairs
 // or more (the matvec path reads an expert once per pair; with fewer pairs per expert it is as
 // fast), within the routing kernel's limits
@@ -835,13 +835,14 @@ scrapgpu_status run_products(Stream * s, const sgk::MatArgs * mats, int n) {
     const int64_t mv_n = matvec_max_n(mats[0]);
     bool fuse = n > 1 && mats[0].N <= mv_n;
     for (int j = 1; j < n && fuse; ++j) {
-        fuse = mats[j].dtype == mats[0].dtype && mats[j].K == mats[0].K && mats[j].x == mats[0].x &&
+        fuse = mats[j].dtype == mats[0].dtype && mats[j].K == mats[0].K && mats[j].nb == mats[0].nb && mats[j].x == mats[0].x &&
                mats[j].ne12 * mats[j].ne13 == 1 && mats[0].ne12 * mats[0].ne13 == 1;
     }
-    // prefill weights of one dtype reading the same x (one slice each): one GEMM launch over all
+    // prefill weights of one dtype and row stride reading the same x (one slice each): one GEMM
+    // launch over all
     bool fuse_mm = n > 1 && mats[0].N > mv_n && mats[0].ne12 * mats[0].ne13 == 1;
     for (int j = 1; j < n && fuse_mm; ++j) {
-        fuse_mm = mats[j].dtype == mats[0].dtype && sgk::matmul_reads_same_x(mats[j], mats[0]) && mats[j].ne12 * mats[j].ne13 == 1;
+        fuse_mm = mats[j].dtype == mats[0].dtype && mats[j].nb == mats[0].nb && sgk::matmul_reads_same_x(mats[j], mats[0]) && mats[j].ne12 * mats[j].ne13 == 1;
     }
     if (fuse_mm) {
         sgk::MatArgs all = mats[0];
@@ -1027,7 +1028,7 @@ bool outputs_apart(const PlanNode * group, int n, const PlanNode & b) {
 }
 
 // consecutive MUL_MAT_ID nodes of a plan that may share one launch: the same x and ids, experts
-// of one dtype, K, count and stride, outputs of one layout apart from every tensor of the group
+// of one dtype, K, count, row and expert stride, outputs of one layout apart from every tensor of the group
 // (outputs_apart), all on the decode path; or, all on the grouped path, one x pre-pass and
 // routing (mul_mat_id_same_x), after which each node runs its GEMM
 bool id_fusable(const PlanNode * group, int n, const PlanNode & b, int cu_count) {
@@ -1048,7 +1049,7 @@ bool id_fusable(const PlanNode * group, int n, const PlanNode & b, int cu_count)
         if (ma.dtype != mb.dtype || ia.n_exp != ib.n_exp || ia.n_used != ib.n_used || !sgk::mul_mat_id_same_x(ma, mb, ia, cu_count)) return false;
         return outputs_apart(group, n, b);
     }
-    if (ma.dtype != mb.dtype || ma.K != mb.K || ma.w_s2 != mb.w_s2 || ia.n_exp != ib.n_exp || ia.n_used != ib.n_used) return false;
+    if (ma.dtype != mb.dtype || ma.K != mb.K || ma.nb != mb.nb || ma.w_s2 != mb.w_s2 || ia.n_exp != ib.n_exp || ia.n_used != ib.n_used) return false;
     if (ma.y_s1 != mb.y_s1 || ma.y_s2 != mb.y_s2) return false;
     return outputs_apart(group, n, b);
 }

@@ -2324,7 +2324,7 @@ hipError_t launch_matmul_mfma(const MatArgs * mats, int nmat, uint8_t * scratch,
     // of all their rows for its shape choice and scratch
     MatArgs a = mats[0];
     for (int j = 1; j < nmat; ++j) {
-        if (mats[j].dtype != a.dtype || !matmul_reads_same_x(mats[j], a) || mats[j].ne12 * mats[j].ne13 != 1 || a.ne12 * a.ne13 != 1) return hipErrorInvalidValue;
+        if (mats[j].dtype != a.dtype || mats[j].nb != a.nb || !matmul_reads_same_x(mats[j], a) || mats[j].ne12 * mats[j].ne13 != 1 || a.ne12 * a.ne13 != 1) return hipErrorInvalidValue;
         a.M += mats[j].M;
     }
     if (is_float_weight(a.dtype) && !float_gemm(a)) return launch_matvec_float(mats, nmat, cu_count, stream, kernel_name, nullptr);

@@ -404,7 +404,7 @@ hipError_t launch_matmul_f32(const MatArgs * mats, int nmat, int cu_count, hipSt
     A.nmat = nmat;
     int64_t rows = 0;
     for (int j = 0; j < nmat; ++j) {
-        if (mats[j].dtype != a.dtype || mats[j].K != a.K || mats[j].N != a.N || (nmat > 1 && mats[j].ne12 * mats[j].ne13 != 1)) return hipErrorInvalidValue;
+        if (mats[j].dtype != a.dtype || mats[j].K != a.K || mats[j].nb != a.nb || mats[j].N != a.N || (nmat > 1 && mats[j].ne12 * mats[j].ne13 != 1)) return hipErrorInvalidValue;
         rows += mats[j].M;
     }
     const int64_t slices = a.ne12 * a.ne13;

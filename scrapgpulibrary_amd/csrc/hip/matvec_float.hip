@@ -210,7 +210,7 @@ hipError_t launch_matvec_float(const MatArgs * mats, int nmat, int cu_count, hip
     A.mt[0] = 0;
     for (int j = 0; j < 3; ++j) {
         const bool has = j < nmat;
-        if (has && (mats[j].dtype != a.dtype || mats[j].K != a.K || mats[j].N != a.N || (nmat > 1 && id == nullptr && mats[j].ne12 * mats[j].ne13 != 1))) {
+        if (has && (mats[j].dtype != a.dtype || mats[j].K != a.K || mats[j].nb != a.nb || mats[j].N != a.N || (nmat > 1 && id == nullptr && mats[j].ne12 * mats[j].ne13 != 1))) {
             return hipErrorInvalidValue;
         }
         A.wm[j] = has ? mats[j].w : nullptr;
