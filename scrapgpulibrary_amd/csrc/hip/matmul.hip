@@ -1911,7 +1911,8 @@ MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
         const int64_t tw = (a.M + 383) / 384 * ((a.N + 127) / 128) * slices;
         const bool wide = free_choice && a.N >= 128 && (a.N + 127) / 128 * 128 * 8 <= 9 * a.N && (a.M % 384 == 0 || a.M >= 8 * 384);
         const bool wide1 = wide && (tw % cu_count == 0 || tw >= 4 * (int64_t) cu_count);
-        const bool wide2 = wide && !wide1 && slices == 1 && tw * 2 <= cu_count && 3 * tw * 2 >= 2 * cu_count && stages / 2 >= 16;
+        const auto fits = [&](int sp) { return !lean || sp == 1 || part_offset(a) + part_bytes(a, sp) <= kLeanBytes; };
+        const bool wide2 = wide && !wide1 && slices == 1 && tw * 2 <= cu_count && 3 * tw * 2 >= 2 * cu_count && stages / 2 >= 16 && fits(2);
         // 192- or 128-row tiles: K past 1024 (shorter K is mostly prologue: 24536x1024 at 500 tokens
         // 59.8 us against 55.2 in 384-row tiles) and at least 8 tiles. Faster as well, but left on
         // the forms that are pinned for them: K up to 1024 in general (4096x512 at 512 tokens 12.1
@@ -1923,7 +1924,7 @@ MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
             float best = 0.0f;
             for (const int rows : {128, 192})
                 for (const int sp : {1, 2, 4}) {
-                    if (stages / sp < 4 || (lean && sp > 1 && part_offset(a) + part_bytes(a, sp) > kLeanBytes)) continue;
+                    if (stages / sp < 4 || !fits(sp)) continue;
                     const float us = lds_gemm_us(a, rows, sp, cu_count);
                     if (c.lds == 0 || us < best) best = us, c.lds = rows, c.split = sp;
                 }
@@ -1961,7 +1962,7 @@ MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
             return c;
         }
         auto cost = [&](int sp) { return (tiles * sp + cu_count - 1) / cu_count * ((stages + sp - 1) / sp + 4); };
-        for (int sp = 2; sp <= 8 && stages / sp >= 8; ++sp)
+        for (int sp = 2; sp <= 8 && stages / sp >= 8 && fits(sp); ++sp)
             if (cost(sp) < cost(c.split)) c.split = sp;
         return c;
     }

@@ -177,3 +177,29 @@ def test_static_scratch_float_weights(hip):
         e = float(np.sum((y_static.astype(np.float64) - ref) ** 2) / np.sum(ref.astype(np.float64) ** 2))
         assert e <= (1e-10 if N == 1 else 1e-6), f"N={N}: NMSE {e:.3e}"
     wb.free()
+
+
+@pytest.mark.parametrize("K,M,N,plain,static", [
+    (4096, 12288, 380, "gemm wide w=12 kg=1 bn=128 rg=1 split=2 lds", "gemm lds w=8 kg=2 bn=128 rows=192 split=1"),
+    (12288, 1500, 700, "gemm lds w=8 kg=2 bn=128 rows=192 split=4", "gemm lds w=8 kg=2 bn=128 rows=128 split=2"),
+    (10240, 4096, 640, "gemm lds w=8 kg=2 bn=128 rows=192 split=2", "gemm lds w=8 kg=2 bn=128 rows=128 split=1"),
+], ids=["384_rows", "4_to_2", "2_to_1"])
+def test_static_scratch_float_splits(hip, K, M, N, plain, static):
+    """F16 prefill whose K splits' partial sums would not fit beside x: fewer splits, not a refusal.
+    Both entry points against the oracle on a sample of rows (f16 operands: x rounded once, NMSE at
+    most 2^-22 / 3)."""
+    dev, st = hip
+    w = O.normal(M * K, 1560, 0.0, 0.02).astype(np.float16).view(np.uint16).reshape(M, K)
+    wb = dev.alloc(w.nbytes)
+    st.write(wb, 0, w.view(np.uint8).reshape(-1))
+    wt = sg.tdesc(sg.F16, (K, M), wb)
+    x = O.normal(N * K, 1561).reshape(N, K)
+    rows = np.unique(np.concatenate([np.arange(0, M, 67), np.arange(M - 40, M)]))
+    ref = O.mul_mat(sg.F16, np.ascontiguousarray(w[rows]), K, len(rows), x, threads=8)
+    for is_static, form in ((True, static), (False, plain)):
+        y = _run(dev, st, wt, x, M, is_static)
+        if dev.info().compute_units == 256:
+            assert sg.last_launch()[0] == form
+        e = float(np.sum((y[:, rows].astype(np.float64) - ref) ** 2) / np.sum(ref.astype(np.float64) ** 2))
+        assert e <= 1e-6, f"NMSE {e:.3e}"
+    wb.free()
