@@ -11,9 +11,12 @@
 // Both read their operands straight from memory into the MFMA's lanes; the waves of a work-group
 // take disjoint steps of K and meet once, in LDS, to add their sums in a fixed tree.
 //
-// Summation: no chain is longer than 8 products before it is added to a longer sum, so the error
-// against 64-bit products is that of the vector kernel (F16 12288x4096 at 8 columns 9.6e-8 against
-// 1.1e-7, F32 128x2048 at 512 columns 1.0e-7 against 0.9e-7, 512x8192 1.1e-7 against 1.3e-7).
+// Summation: no chain is longer than 8 products before it is added to a longer sum, and the waves'
+// sums are added in 64 bits and rounded once, so the error against 64-bit products is below that of
+// the vector kernel, which it must not exceed (activations with one channel in 64 eight times larger;
+// F16 4096x4096 at 8 columns 8.7e-8 against 1.06e-7, 12288x2056 at 300 8.0e-8 against 9.3e-8, F32
+// 128x2048 at 512 8.1e-8 against 9.2e-8, 512x8192 at 2048 1.09e-7 against 1.27e-7; with the waves'
+// sums added in f32 it was up to 6% above it at K of 500 to 2100).
 #include "kernels.h"
 #include "weight_float.h"
 
@@ -189,10 +192,10 @@ __global__ __launch_bounds__(512) void k_mvq(MmfArgs A) {
     __syncthreads();
     if (threadIdx.x < 4 * V) {
         const int t = threadIdx.x;
-        float p[W];
+        double p[W];
 #pragma unroll
         for (int k = 0; k < W; ++k) p[k] = red[k][t];
-        const float sum = tree<W>(p);
+        const float sum = (float) tree<W>(p);
         const int c = (t >> 4) % C, r = (t >> 4) / C;
         const int64_t m = m0 + 4 * r + (t & 3), n = n0 + 4 * c + ((t >> 2) & 3);
         if (m < P.M && n < N) P.y[n * P.ys1 + m] = sum;
@@ -208,8 +211,9 @@ __global__ __launch_bounds__(512) void k_mvq(MmfArgs A) {
 // launches of 8 columns: F32 128x2048 at 512 columns 9.5 us (16 x 16 tiles) against 965; 500x4096 at
 // 512 32 us (32 x 32; 58.7 in 16 x 16); 4096x4096 at 512 230 us = 75 TFLOP/s of 157 (64 x 32) against
 // 2519; F16 2500x520 at 500 40 us (32 x 32) against 169 for the vector kernel in one launch. Chains of
-// 2 MFMAs added in a tree of 4 are faster on large tiles (192 and 30 us) but their error is larger
-// than the vector kernel's at short K (256x1024 9.5e-8 against 8.7e-8).
+// 2 MFMAs added in a tree of 4 are faster on large tiles (192 and 30 us) but their error was larger
+// than the vector kernel's at short K (256x1024 9.5e-8 against 8.7e-8, with the waves' sums added in
+// f32).
 constexpr int kRun = 4; // steps per run of the two-level sum
 
 template <int WT, int R, int C, int W, bool XV>
@@ -231,8 +235,11 @@ __global__ __launch_bounds__(64 * W) void k_mmf(MmfArgs A) {
     for (int c = 0; c < C; ++c) col[c] = P.x + min<int64_t>(n0 + 16 * c + i, N - 1) * A.a.x_s1;
 
     // the lane's elements of a step: two groups of 4, each 16 bytes of F32, or 16 bytes of F16 / BF16
-    // together, so that the four parts of a row read one run of 64 bytes per load
-    const int o0 = WT == F32 ? 4 * q : 8 * q, o1 = WT == F32 ? 16 + 4 * q : 8 * q + 4;
+    // together, so that the four parts of a row read one run of 64 bytes per load. (The parts in
+    // descending order: an MFMA adds its 4 products one after the other, so the first is rounded four
+    // times and the last once. Random data do not care; with large activations in a step's first part
+    // this order has the smaller error, F16 64x64 6.3e-8 against 7.0e-8.)
+    const int g = 3 - q, o0 = WT == F32 ? 4 * g : 8 * g, o1 = WT == F32 ? 16 + 4 * g : 8 * g + 4;
     struct Raw {
         uint4 w[R][S][WT == F32 ? 2 : 1];
         float4 x[C][S][2];
@@ -330,10 +337,10 @@ __global__ __launch_bounds__(64 * W) void k_mmf(MmfArgs A) {
             for (int e = 0; e < 4; ++e) red[wave][(r * C + c) * 4 + e][lane] = tot[r][c][e] + run[r][c][e];
     __syncthreads();
     for (int v = wave; v < V; v += W) {
-        float p[W];
+        double p[W];
 #pragma unroll
         for (int h = 0; h < W; ++h) p[h] = red[h][v][lane];
-        const float sum = tree<W>(p);
+        const float sum = (float) tree<W>(p);
         const int r = v / (4 * C), c = v / 4 % C, e = v % 4;
         const int64_t m = m0 + 16 * r + i, t = n0 + 16 * c + 4 * q + e;
         if (m < P.M && t < N) P.y[t * P.ys1 + m] = sum;

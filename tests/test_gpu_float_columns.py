@@ -102,3 +102,21 @@ def test_float_columns_non_finite(hip, dtype, K, M, N):
     assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
     ok = np.isfinite(ref)
     assert np.array_equal(y[~ok & ~np.isnan(ref)], ref[~ok & ~np.isnan(ref)]) and nmse(y[ok], ref[ok]) <= bound(K)
+
+
+@pytest.mark.parametrize("dtype,K,M,N", [(sg.BF16, 520, 4096, 5), (sg.F16, 4096, 3072, 8), (sg.F16, 1000, 1000, 64), (sg.BF16, 2056, 1500, 40),
+                                         (sg.F32, 512, 512, 1100), (sg.F32, 1024, 300, 128), (sg.F16, 64, 1000, 30)], ids=lambda v: str(v))
+def test_float_columns_error(hip, dtype, K, M, N):
+    """The error against 64-bit products is no larger than the vector kernel's (1 and 2 columns per call),
+    on activations with outlier channels."""
+    dev, st = hip
+    wbytes, wf = float_weights(dtype, M, K, 8300 + K)
+    x = O.normal(N * K, 8301 + N).reshape(N, K)
+    x[:, 5::64] *= 8
+    exact = x.astype(np.float64) @ wf.astype(np.float64).T
+    y = run(dev, st, dtype, wbytes, K, M, x, check_form=False)
+    assert sg.last_launch()[0].startswith("float mfma") or dev.info().compute_units != 256, sg.last_launch()
+    cols = np.arange(N) if N <= 64 else np.linspace(0, N - 1, 64).astype(int)  # (a sample: some 30000 values differ by 1% in their mean error)
+    v = np.concatenate([run(dev, st, dtype, wbytes, K, M, x[cols[i:i + 2]]) for i in range(0, len(cols), 2)])
+    e, ev = nmse(y, exact) ** 0.5, nmse(v, exact[cols]) ** 0.5
+    assert e <= ev, f"{IDS[dtype]} {M}x{K} N={N}: {e:.3e}, the vector kernel {ev:.3e}"
