@@ -478,29 +478,34 @@ __device__ __forceinline__ uint2 ga_tile(int expert, int first, int count) {
     return make_uint2((uint32_t) first, (uint32_t) expert << 8 | (uint32_t) count);
 }
 
-// Index arithmetic ahead of a kernel's first load. A 64-bit division is tens of dependent
-// instructions (a call over few tokens has up to ten of them before it asks for its first weights),
-// so a quotient that the usual call knows, 0 or 1 for one slice and one split, is not divided for,
-// and tile numbers (the grid's x extent) are divided in 32 bits.
+// Index arithmetic ahead of a kernel's first load: quotients that the usual call knows, 0 or 1 for
+// one slice and one split, are not divided for, and the others are divided in 32 bits (at most 65535
+// slices, x rows below 2^31 in all, tile numbers in the grid's x extent, K below 2^31). A 64-bit
+// division is a hundred instructions: up to ten of them stood ahead of a call's first weights, and
+// even those that are jumped over spread a kernel's entry over more cache lines of code (Q6_K
+// 166+2836+346 rows x 1536 at 20 tokens 10.16 us with them, 10.26 with them behind branches, 10.24 in
+// 32 bits, 9.65 with pick3 as well; 3348 rows in one weight 10.40, 10.37, 10.30 and 9.65).
 struct Slice {
     int64_t i2, i3;
 };
-__device__ __forceinline__ Slice slice_of(const MatArgs & a, int64_t sl) { // x slice sl
+__device__ __forceinline__ Slice slice_of(const MatArgs & a, uint32_t sl) { // x slice sl
     if (sl == 0) return {0, 0};
-    const int64_t i3 = sl / a.ne12;
-    return {sl - i3 * a.ne12, i3};
+    const uint32_t n = (uint32_t) a.ne12, i3 = sl / n;
+    return {(int64_t) (sl - i3 * n), (int64_t) i3};
 }
 __device__ __forceinline__ int64_t slice_w(const MatArgs & a, const Slice & c) { // its weights' byte offset
     int64_t o = 0;
-    if (c.i2 != 0) o += (int64_t) ((uint64_t) (c.i2 / a.r2) * a.w_s2);
-    if (c.i3 != 0) o += (int64_t) ((uint64_t) (c.i3 / a.r3) * a.w_s3);
+    if (c.i2 != 0) o += (int64_t) ((uint32_t) c.i2 / (uint32_t) a.r2 * a.w_s2);
+    if (c.i3 != 0) o += (int64_t) ((uint32_t) c.i3 / (uint32_t) a.r3 * a.w_s3);
     return o;
 }
-__device__ __forceinline__ int64_t row_slice(int64_t row, int64_t n) { return row < n ? 0 : row / n; } // the slice of x row `row`
+__device__ __forceinline__ uint32_t row_slice(int64_t row, int64_t n) { // the slice of x row `row`
+    return row < n ? 0 : (uint32_t) row / (uint32_t) n;
+}
 // the first stage of a split (K in groups of 4 stages; split = n: K's end, or up to 3 past it)
 __device__ __forceinline__ int64_t split_start(int64_t groups, int split, int n) {
     if (split == 0) return 0;
-    return 4 * (split == n ? groups : groups * split / n);
+    return 4 * (split == n ? groups : (int64_t) ((uint32_t) groups * (uint32_t) split / (uint32_t) n));
 }
 struct TileOf {
     int64_t tm, tn;
@@ -539,6 +544,14 @@ struct MmArgs {
     float * ym[3];
     int64_t ys1m[3];
 };
+
+// entry j of a table of MmArgs, selected from all three: their loads go out with a kernel's first ones,
+// while an index makes an address that waits for it (another round trip ahead of the first weights)
+template <typename T>
+__device__ __forceinline__ T pick3(const T * v, int j) {
+    const T a = v[0], b = v[1], c = v[2];
+    return j == 0 ? a : j == 1 ? b : c;
+}
 
 // padded x tile rows (the wide GEMM): 16-byte chunk c of token n at n * XR + 8 c (f16). The 16
 // bytes of padding put consecutive tokens 4 banks apart, so the 16 lanes of one ds_read_b128
@@ -679,15 +692,15 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     const Slice slc = slice_of(L.a, sl);
     // the wave's matrix (several when weights share x)
     const int64_t grow = tm * BMT + 32 * RG * wave; // packed: the wave's first row over all matrices
-    const int mj = L.nmat == 1 ? 0
-                 : L.packed    ? min(L.nmat - 1, grow >= L.mo[1] ? (grow >= L.mo[2] ? 2 : 1) : 0)
-                               : (tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0);
-    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + slice_w(L.a, slc);
+    const int mj = GA ? 0
+                 : L.packed ? min(L.nmat - 1, grow >= L.mo[1] ? (grow >= L.mo[2] ? 2 : 1) : 0)
+                            : (tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0);
+    const uint8_t * w = GA ? L.a.w : pick3(L.wm, mj) + slice_w(L.a, slc);
     const int64_t K = L.a.K, nb = L.a.nb;
-    const int64_t M = L.nmat > 1 ? L.Mm[mj] : L.a.M;
+    const int64_t M = GA ? L.a.M : pick3(L.Mm, mj);
     int64_t N = L.a.N;
     int64_t n0 = tn * BN;
-    const int64_t m0 = L.packed ? grow - L.mo[mj] : (tm - L.mt[mj]) * BMT + 32 * RG * wave;
+    const int64_t m0 = GA ? grow : L.packed ? grow - pick3(L.mo, mj) : (tm - pick3(L.mt, mj)) * BMT + 32 * RG * wave;
     int32_t * ga_rows = reinterpret_cast<int32_t *>(lds_mm + KG * 2 * BN * BK); // GA: x row of tile token n
     int64_t * ga_y = reinterpret_cast<int64_t *>(ga_rows + BN);               // GA: its y element offset
     int32_t ga_cnt = BN;                                                      // GA: the tile's pairs
@@ -956,11 +969,11 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     float * y;
     int64_t ys1;
     if (L.split == 1) {
-        y = L.nmat > 1 ? L.ym[mj] : L.a.y + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
-        ys1 = L.nmat > 1 ? L.ys1m[mj] : L.a.y_s1;
+        y = GA ? L.a.y : pick3(L.ym, mj) + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
+        ys1 = GA ? L.a.y_s1 : pick3(L.ys1m, mj);
     } else {
         const int64_t mt_all = L.mo[L.nmat]; // the partials' row length: all matrices' rows
-        y = L.part + ((uint64_t) split * slices + (uint64_t) sl) * N * mt_all + L.mo[mj];
+        y = L.part + ((uint64_t) split * slices + (uint64_t) sl) * N * mt_all + pick3(L.mo, mj);
         ys1 = mt_all;
     }
     const float * xs = L.xs + (uint64_t) sl * N;
@@ -1385,12 +1398,12 @@ __global__ __launch_bounds__(64 * KW * RW) void k_gemm_n(MmArgs L) {
     // the wave's R32 group (past the last one: the last one again, not stored)
     const int64_t tm = min<int64_t>((int64_t) blockIdx.x * RW + rw, L.tiles_m - 1), sl = blockIdx.y;
     const bool live = (int64_t) blockIdx.x * RW + rw < L.tiles_m;
-    const Slice slc = slice_of(L.a, sl);
-    const int mj = L.nmat == 1 ? 0 : (tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0);
-    const uint8_t * w = L.nmat > 1 ? L.wm[mj] : L.a.w + slice_w(L.a, slc);
+    const Slice slc = slice_of(L.a, sl); // (several matrices: slice 0)
+    const int mj = tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0;
+    const uint8_t * w = pick3(L.wm, mj) + slice_w(L.a, slc);
     const int64_t nb = L.a.nb, N = L.a.N;
-    const int64_t M = L.nmat > 1 ? L.Mm[mj] : L.a.M;
-    const int64_t m0 = (tm - L.mt[mj]) * 32;
+    const int64_t M = pick3(L.Mm, mj);
+    const int64_t m0 = (tm - pick3(L.mt, mj)) * 32;
     const int S = (int) L.stages, U = (S + 1) / 2; // units of 2 stages (the K-quants' blocks)
     const int s0 = 2 * (U * kw / KW), s1 = min(2 * (U * (kw + 1) / KW), S), lim = max(s1 - 1, 0);
 
@@ -1477,8 +1490,8 @@ __global__ __launch_bounds__(64 * KW * RW) void k_gemm_n(MmArgs L) {
         if (r > 1) __syncthreads();
     }
     if (kw != 0 || !live) return;
-    float * y = L.nmat > 1 ? L.ym[mj] : L.a.y + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
-    const int64_t ys1 = L.nmat > 1 ? L.ys1m[mj] : L.a.y_s1;
+    float * y = pick3(L.ym, mj) + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
+    const int64_t ys1 = pick3(L.ys1m, mj);
     const float * xs = L.xs + (uint64_t) sl * N;
     const int64_t m = m0 + j;
 #pragma unroll
@@ -1496,7 +1509,9 @@ __global__ __launch_bounds__(64 * KW * RW) void k_gemm_n(MmArgs L) {
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_split_reduce(MmArgs L) {
     const int64_t N = L.a.N, Mt = L.mo[L.nmat];
-    const int64_t row = blockIdx.x, sl = row_slice(row, N), n = row - sl * N;
+    const int64_t row = blockIdx.x;
+    const uint32_t sl = row_slice(row, N);
+    const int64_t n = row - sl * N;
     const Slice slc = slice_of(L.a, sl);
     const uint64_t plane = (uint64_t) L.a.ne12 * L.a.ne13 * N * Mt;
     const float * p = L.part + row * Mt;
@@ -1603,7 +1618,8 @@ __device__ __forceinline__ void x_row_to_f16(const MatArgs & a, uint16_t * xb, f
                                              int tid, float * wmax, bool live) {
     constexpr int kCached = 6; // K <= 12288 is read once (TPR = 64: 3072)
     constexpr int STEP = 8 * TPR;
-    const int64_t sl = row_slice(row, a.N), n = row - sl * a.N;
+    const uint32_t sl = row_slice(row, a.N);
+    const int64_t n = row - sl * a.N;
     const Slice slc = slice_of(a, sl);
     const float * xp = a.x + slc.i2 * a.x_s2 + slc.i3 * a.x_s3 + n * a.x_s1;
     uint16_t * op = xb + row * a.K;
