@@ -11,12 +11,13 @@
 // Both read their operands straight from memory into the MFMA's lanes; the waves of a work-group
 // take disjoint steps of K and meet once, in LDS, to add their sums in a fixed tree.
 //
-// Summation: no chain is longer than 8 products before it is added to a longer sum, and the waves'
-// sums are added in 64 bits and rounded once, so the error against 64-bit products is below that of
-// the vector kernel, which it must not exceed (activations with one channel in 64 eight times larger;
-// F16 4096x4096 at 8 columns 8.7e-8 against 1.06e-7, 12288x2056 at 300 8.0e-8 against 9.3e-8, F32
-// 128x2048 at 512 8.1e-8 against 9.2e-8, 512x8192 at 2048 1.09e-7 against 1.27e-7; with the waves'
-// sums added in f32 it was up to 6% above it at K of 500 to 2100).
+// Summation: no chain is longer than 8 products before it is added to a longer sum, and pairs of the
+// waves' sums are added in 64 bits and rounded once, so the error against 64-bit products is below that
+// of the vector kernel, which it must not exceed (activations with one channel in 64 eight times
+// larger; F16 4096x4096 at 8 columns 9.2e-8 against 1.06e-7, 12288x2056 at 300 8.5e-8 against 9.3e-8,
+// F32 128x2048 at 512 8.8e-8 against 9.2e-8, 512x512 at 1024 7.9e-8 against 8.2e-8, 512x8192 at 2048
+// 1.10e-7 against 1.27e-7; with the waves' sums added in f32 it was up to 6% above it at K of 500 to
+// 2100).
 #include "kernels.h"
 #include "weight_float.h"
 
@@ -73,6 +74,16 @@ __device__ __forceinline__ T tree(T (&p)[W]) {
 #pragma unroll
         for (int k = 0; k + h < W; k += 2 * h) p[k] += p[k + h];
     return p[0];
+}
+
+// the sum of the W waves' values at(wave): pairs in 32 bits, those in 64, rounded once (all in 64 bits
+// the error is 5% lower, but F16 8192x128 at 4 columns, 64 slices took 94.4 us against 93.8, and 93.0 all in 32)
+template <int W, typename F>
+__device__ __forceinline__ float sum_waves(F at) {
+    double p[W / 2];
+#pragma unroll
+    for (int k = 0; k < W / 2; ++k) p[k] = at(2 * k) + at(2 * k + 1);
+    return (float) tree<W / 2>(p);
 }
 
 // reduce-scatter of V values over the 16 lanes that share lane % 4 (lanes 4 b + j): afterwards lane
@@ -192,10 +203,7 @@ __global__ __launch_bounds__(512) void k_mvq(MmfArgs A) {
     __syncthreads();
     if (threadIdx.x < 4 * V) {
         const int t = threadIdx.x;
-        double p[W];
-#pragma unroll
-        for (int k = 0; k < W; ++k) p[k] = red[k][t];
-        const float sum = (float) tree<W>(p);
+        const float sum = sum_waves<W>([&](int k) { return red[k][t]; });
         const int c = (t >> 4) % C, r = (t >> 4) / C;
         const int64_t m = m0 + 4 * r + (t & 3), n = n0 + 4 * c + ((t >> 2) & 3);
         if (m < P.M && n < N) P.y[n * P.ys1 + m] = sum;
@@ -238,8 +246,9 @@ __global__ __launch_bounds__(64 * W) void k_mmf(MmfArgs A) {
     // together, so that the four parts of a row read one run of 64 bytes per load. (The parts in
     // descending order: an MFMA adds its 4 products one after the other, so the first is rounded four
     // times and the last once. Random data do not care; with large activations in a step's first part
-    // this order has the smaller error, F16 64x64 6.3e-8 against 7.0e-8.)
-    const int g = 3 - q, o0 = WT == F32 ? 4 * g : 8 * g, o1 = WT == F32 ? 16 + 4 * g : 8 * g + 4;
+    // this order has the smaller error, F16 64x64 6.3e-8 against 7.0e-8. F32 keeps the ascending order,
+    // 128x2048 at 512 columns 9.6 us against 9.8.)
+    const int g = WT == F32 ? q : 3 - q, o0 = WT == F32 ? 4 * g : 8 * g, o1 = WT == F32 ? 16 + 4 * g : 8 * g + 4;
     struct Raw {
         uint4 w[R][S][WT == F32 ? 2 : 1];
         float4 x[C][S][2];
@@ -337,10 +346,18 @@ __global__ __launch_bounds__(64 * W) void k_mmf(MmfArgs A) {
             for (int e = 0; e < 4; ++e) red[wave][(r * C + c) * 4 + e][lane] = tot[r][c][e] + run[r][c][e];
     __syncthreads();
     for (int v = wave; v < V; v += W) {
-        double p[W];
+        // (as sum_waves, one after the other; 4 waves' sums all in 64 bits. K of two units has no more than
+        // two waves' sums: without the branch 500x64 at 100 columns, 64 slices 59.3 us against 56.1, 2500x72
+        // at 300 columns 14.0 against 13.3; not for F32, whose 512x512 at 1024 columns took 13.5 us with
+        // such a branch against 13.1)
+        constexpr int PW = W > 4 ? 2 : 1;
+        const auto part = [&](int h) { return PW == 2 ? red[h][v][lane] + red[h + 1][v][lane] : red[h][v][lane]; };
+        double s = part(0);
+        if (WT == F32 || K > PW * KU) {
 #pragma unroll
-        for (int h = 0; h < W; ++h) p[h] = red[h][v][lane];
-        const float sum = (float) tree<W>(p);
+            for (int h = PW; h < W; h += PW) s += part(h);
+        }
+        const float sum = (float) s;
         const int r = v / (4 * C), c = v / 4 % C, e = v % 4;
         const int64_t m = m0 + 16 * r + i, t = n0 + 16 * c + 4 * q + e;
         if (m < P.M && t < N) P.y[t * P.ys1 + m] = sum;
