@@ -1742,7 +1742,7 @@ __global__ __launch_bounds__(256) void k_x_to_f16(MatArgs a, uint16_t * xb, floa
 // pairs p = t * n_used + slot grouped by expert (ids clamped to [0, E)), and per token tile (bn
 // pairs) its expert, first pair and count, 0 past the last tile. Counts with LDS atomics,
 // exclusive scans of the counts and of the tile counts (one expert per thread, wave scans), each
-// expert's tiles written by its thread, then each pair placed at its expert's cursor (its id read
+// expert's tiles written by its thread or its wave, then each pair placed at its expert's cursor (its id read
 // again: it is in the L2 by then). The order
 // of the pairs inside an expert follows the LDS atomics; no output depends on it (each is one
 // pair's own sum over K).
@@ -1791,7 +1791,18 @@ __device__ __forceinline__ void moe_route(const RouteArgs & r) {
     cur[tid] = ea;
     int total = 0; // token tiles of all experts
     for (int w2 = 0; w2 < 16; ++w2) total += wsum[1][w2];
-    for (int k = 0; k < tl; ++k) r.tiles[eb + k] = ga_tile(tid, ea + k * r.bn, min(r.bn, c - k * r.bn));
+    const auto tile = [&](int e, int first, int count, int at, int k) __attribute__((always_inline)) {
+        r.tiles[at + k] = ga_tile(e, first + k * r.bn, min(r.bn, count - k * r.bn));
+    };
+    // (an expert of many tiles by its thread's whole wave: one thread's stores follow each other at
+    // some 16 ns, 1000 tiles of one expert of 64000 pairs 16 us in the launch that the GEMM waits for)
+    const bool many = tl > 32;
+    for (int k = 0; !many && k < tl; ++k) tile(tid, ea, c, eb, k);
+    for (uint64_t m = __ballot(many); m != 0; m &= m - 1) {
+        const int l = __builtin_ctzll(m), e = tid - lane + l;
+        const int ec = __shfl(c, l), et = __shfl(tl, l), ef = __shfl(ea, l), at = __shfl(eb, l);
+        for (int k = lane; k < et; k += 64) tile(e, ef, ec, at, k);
+    }
     for (int i = total + tid; i < r.n_tiles; i += 1024) r.tiles[i] = make_uint2(0, 0);
     __syncthreads();
     for (int p = tid; p < P; p += 1024) r.pairs[atomicAdd(&cur[expert(p)], 1)] = (uint16_t) p;

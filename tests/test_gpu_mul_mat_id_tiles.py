@@ -68,3 +68,28 @@ def test_x_rows_by_wave_and_by_group(hip, dtype, K):
     ref = O.mul_mat_id(dtype, w, K, M, E, x, ids)
     d = ((y.astype(np.float64) - ref) ** 2).sum(2) / (ref.astype(np.float64) ** 2).sum(2)
     assert d.max() <= 20 * 5e-5, d.max()
+
+
+def test_experts_of_many_tiles(hip):
+    """Routing far from balanced: experts of more than 32 token tiles (their table is written by a wave) beside
+    experts of few and of none, two of them in one wave; against every token's product with its expert in
+    64 bits."""
+    dev, st = hip
+    K, M, E, T, nu = 256, 40, 130, 14000, 2
+    rng = np.random.default_rng(100)
+    ids = rng.integers(0, E, (T, nu)).astype(np.int32)
+    hot = rng.random((T, nu))
+    for e, lo, hi in ((3, 0.0, 0.3), (60, 0.3, 0.55), (127, 0.55, 0.85)):
+        ids[(hot >= lo) & (hot < hi)] = e
+    ids[ids == 61] = 62  # (no pairs beside the many)
+    w = O.quantize(sg.Q8_0, O.normal(K * M * E, 101, 0.0, 0.02))
+    x = O.normal(T * K, 102).reshape(T, 1, K)
+    y = run_mul_mat_id(dev, st, sg.Q8_0, w, K, M, E, x, ids)
+    deq = O.dequantize(sg.Q8_0, w, K * M * E).reshape(E, M, K).astype(np.float64)
+    ref = np.empty(y.shape)
+    for e in range(E):
+        t, s = np.nonzero(ids == e)
+        ref[t, s] = x[t, 0].astype(np.float64) @ deq[e].T
+    d = ((y - ref) ** 2).sum(2) / (ref ** 2).sum(2)
+    assert d.max() <= 20 * 5e-5, (d.max(), int(d.argmax()))
+    assert ((y - ref) ** 2).sum() <= 5e-5 * (ref ** 2).sum()
