@@ -1870,8 +1870,8 @@ constexpr size_t kLeanBytes = (size_t) 32 << 20;
 // less, as the tiles in flight share the L2s (4096x4096 at 512: half the CUs, 0.37 us a stage), but
 // hardly where every tile streams weights of its own (one token tile: 12288x4096 at 128, 96 tiles,
 // 0.64 us); 6 stages' time of prologue and epilogue; K splits move their partial sums at 4.7 TB/s.
-float lds_gemm_us(const MatArgs & a, int rows, int split, int cu_count) {
-    const int64_t tn = (a.N + 127) / 128, tiles = (a.M + rows - 1) / rows * tn * a.ne12 * a.ne13 * split;
+float lds_gemm_us(const MatArgs & a, int rows, int64_t tiles_m, int split, int cu_count) {
+    const int64_t tn = (a.N + 127) / 128, tiles = tiles_m * tn * a.ne12 * a.ne13 * split;
     const float part = (float) (tiles % cu_count) / (float) cu_count, least = tn == 1 ? 0.75f : tn == 2 ? 0.55f : 0.35f;
     const float rounds = (float) (tiles / cu_count) + (part > 0.0f ? least + (1.0f - least) * part : 0.0f);
     const float us = rounds * ((float) a.K / 64.0f / (float) split + 6.0f) * (rows == 192 ? 0.82f : 0.62f);
@@ -1957,7 +1957,7 @@ MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
             for (const int rows : {128, 192})
                 for (const int sp : {1, 2, 4}) {
                     if (stages / sp < 4 || !fits(sp)) continue;
-                    const float us = lds_gemm_us(a, rows, sp, cu_count);
+                    const float us = lds_gemm_us(a, rows, (a.M + rows - 1) / rows, sp, cu_count);
                     if (c.lds == 0 || us < best) best = us, c.lds = rows, c.split = sp;
                 }
             c.w = 8;
@@ -2292,6 +2292,29 @@ static hipError_t launch_narrow(MmArgs & L, const MatArgs * mats, int nmat, cons
     return hipLaunchKernel(fn, grid, dim3((unsigned) (64 * cfg.kw * cfg.rw)), args, lds, stream);
 }
 
+// Several 16-bit weights sharing x: k_gemm_l tiles each of them on its own, config_of counts tiles over
+// all their rows. Where there are more, the tile's rows, and the K splits up to those that the scratch
+// is for, are chosen again from the tiles there are.
+static void retile(MmConfig & c, const MatArgs & a, const MatArgs * mats, int nmat, int cu_count) {
+    const auto tiles = [&](int rows) {
+        int64_t t = 0;
+        for (int j = 0; j < nmat; ++j) t += (mats[j].M + rows - 1) / rows;
+        return t;
+    };
+    // (four rounds of 384-row tiles or more: the last one's fill hardly counts, 8192+8192+8192 rows x 1024 at
+    // 2000 tokens 150 us against 155)
+    if (tiles(c.lds) == (a.M + c.lds - 1) / c.lds || (c.lds == 384 && c.split == 1 && tiles(384) * ((a.N + 127) / 128) >= 4 * (int64_t) cu_count)) return;
+    const int most = c.split;
+    float best = 0.0f;
+    for (const int rows : {128, 192})
+        for (int sp = 1; sp <= most; sp *= 2) {
+            const float us = lds_gemm_us(a, rows, tiles(rows), sp, cu_count);
+            if (best == 0.0f || us < best) best = us, c.lds = rows, c.split = sp;
+        }
+    c.w = 8;
+    c.kg = 2;
+}
+
 // 16-bit weights with both operands in LDS: L's tiles and row ranges as set by launch_matmul_mfma
 static hipError_t launch_lds(const MmArgs & L, const MmConfig & cfg, hipStream_t stream, const char ** kernel_name) {
     const MatArgs & a = L.a;
@@ -2369,7 +2392,8 @@ hipError_t launch_matmul_mfma(const MatArgs * mats, int nmat, uint8_t * scratch,
     const int64_t xsum_row = xsum_row_of(a);
     if (rows > 0x7fffffff) return hipErrorInvalidValue;
     const dim3 xg((unsigned) rows);
-    const MmConfig cfg = config_of(a, cu_count, lean);
+    MmConfig cfg = config_of(a, cu_count, lean);
+    if (nmat > 1 && cfg.lds != 0) retile(cfg, a, mats, nmat, cu_count);
     if (x_ready) {
         // x converted by the previous product's pre-pass (matmul_same_x)
     } else if (cfg.narrow) {

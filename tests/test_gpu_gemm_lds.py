@@ -69,3 +69,68 @@ def test_gemm_lds_multi_and_slices(hip, dtype, K, Ms, N, S):
             assert nmse(y[s], ref) <= PREFILL_NMSE[dtype], (M, s)
     for b in bufs:
         b.free()
+
+
+@pytest.mark.parametrize("dtype,K,M,N,form", [
+    (sg.F16, 1152, 1000, 130, "gemm lds w=8 kg=2 bn=128 rows=128"),                # tails in rows, tokens and stages
+    (sg.BF16, 4224, 12290, 380, "gemm wide w=12 kg=1 bn=128 rg=1 split=2 lds"),    # K in splits
+    (sg.F16, 1280, 12288, 511, "gemm lds w=8 kg=2 bn=128 rows=192 split=1"),
+], ids=["128_rows", "384_rows_split", "192_rows"])
+def test_gemm_lds_non_finite(hip, dtype, K, M, N, form):
+    """Inf and NaN in x and weights reach exactly the outputs that they reach in the reference: the last row
+    and token, which the tiles' padding reads again, hold some of them."""
+    dev, st = hip
+    wbytes, _ = float_weights(dtype, M, K, 9200)
+    x = O.normal(N * K, 9201).reshape(N, K)
+    x[N - 1, K - 1], x[N - 2, 0], x[3, 64] = np.inf, np.nan, -np.inf
+    w = np.ascontiguousarray(wbytes).view(np.uint16).reshape(M, K).copy()
+    inf, nan = (0x7C00, 0x7E00) if dtype == sg.F16 else (0x7F80, 0x7FC0)
+    w[M - 1, K - 2], w[M - 2, 1], w[7, 65] = inf, nan, inf
+    y = run(dev, st, dtype, w, K, M, x, check_form=False)
+    if dev.info().compute_units == 256:
+        assert sg.last_launch()[0].startswith(form), sg.last_launch()
+    rows = np.unique(np.concatenate([np.arange(0, M, max(1, M // 300)), [7, 8], np.arange(M - 130, M)]))
+    ref = O.mul_mat(dtype, np.ascontiguousarray(w[rows]), K, len(rows), x, threads=8)
+    y = y[:, rows]
+    assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
+    ok = np.isfinite(ref)
+    bad = ~ok & ~np.isnan(ref)
+    assert bad.any() and np.array_equal(y[bad], ref[bad]) and nmse(y[ok], ref[ok]) <= PREFILL_NMSE[dtype]
+
+
+@pytest.mark.parametrize("Ms,K,N,form", [
+    ((4096, 1024, 1024), 1152, 2048, "gemm lds w=8 kg=2 bn=128 rows=128 split=1"),  # 34 192-row tiles against 32 over all rows: past two rounds of the CUs
+    ((4000, 1100, 1044), 4224, 1000, "gemm lds w=8 kg=2 bn=128 rows="),             # 384-row tiles in two splits would take a second round
+    ((8192, 8192, 8192), 128, 512, "gemm lds w=8 kg=2 bn=128 rows="),               # two stages of K; one round of 384-row tiles over all rows, two apart
+    ((3840, 1152, 1152), 4224, 1000, "gemm wide w=12 kg=1 bn=128 rg=1 split=2 lds"),  # whole 384-row tiles: as one weight
+], ids=["192", "384_split", "384", "whole"])
+def test_gemm_lds_multi_tiles(hip, Ms, K, N, form):
+    """Several weights whose tiles are more than those of their rows together: the tiles chosen for them."""
+    dev, st = hip
+    dtype = sg.BF16
+    x = O.normal(N * K, 9300).reshape(N, K)
+    xb = dev.alloc(x.nbytes)
+    xt = sg.tdesc(sg.F32, (K, N), xb)
+    st.write(xb, 0, x)
+    bufs, wts, yts, ws = [xb], [], [], []
+    for j, M in enumerate(Ms):
+        w = np.ascontiguousarray(float_weights(dtype, M, K, 9301 + j)[0]).view(np.uint16).reshape(M, K)
+        wb, yb = dev.alloc(w.nbytes), dev.alloc(4 * M * N)
+        st.write(wb, 0, w.view(np.uint8).reshape(-1))
+        bufs += [wb, yb]
+        ws.append(w)
+        wts.append(sg.tdesc(dtype, (K, M), wb))
+        yts.append(sg.tdesc(sg.F32, (M, N), yb))
+    op, keep = sg.multi_op(wts, xt, yts)
+    st.execute(op)
+    st.sync()
+    if dev.info().compute_units == 256:
+        assert sg.last_launch()[0].startswith(form), sg.last_launch()
+    cols = np.unique(np.concatenate([np.arange(0, N, 37), np.arange(N - 20, N)]))
+    for M, yt, w in zip(Ms, yts, ws):
+        rows = np.unique(np.concatenate([np.arange(0, M, 61), np.arange(M - 70, M)]))
+        ref = O.mul_mat(dtype, np.ascontiguousarray(w[rows]), K, len(rows), np.ascontiguousarray(x[cols]), threads=8)
+        y = st.download(yt).reshape(N, M)[np.ix_(cols, rows)]
+        assert nmse(y, ref) <= PREFILL_NMSE[dtype], M
+    for b in bufs:
+        b.free()
