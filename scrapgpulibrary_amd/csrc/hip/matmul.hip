@@ -1952,7 +1952,13 @@ MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
         // 29.1) and a part-empty token tile in the 384-row form's K splits (12288x4096 at 380 tokens
         // 60 against 80 us; 96 before its weights went through LDS)
         const int64_t tn = (a.N + 127) / 128;
-        if (free_choice && a.N > 64 && a.K > 1024 && (a.M + 127) / 128 * tn * slices >= 8 && !(wide2 && a.N % 128 != 0)) {
+        // K of 512 to 1024 as well where the 4-wave form's 128 x 128 tiles, two per CU at a time, leave a last
+        // round at most half full: with x and weights in plain order that form got 1 to 6% slower there (BF16
+        // 9000x640 at 1024 tokens 46.1 -> 47.5 us, 28672x1024 at 300 54.2 -> 57.8), and k_gemm_l takes 37.7
+        // and 36.4. Not with a fuller last round: 65000x512 at 256 tokens 55.5 us against 51.9
+        const int64_t tiles128 = (a.M + 127) / 128 * tn * slices, last = tiles128 % (2 * (int64_t) cu_count);
+        const bool ragged = a.K >= 512 && !wide1 && tiles128 > 2 * (int64_t) cu_count && last > 0 && last <= cu_count;
+        if (free_choice && a.N > 64 && (a.K > 1024 || ragged) && tiles128 >= 8 && !(wide2 && a.N % 128 != 0)) {
             float best = 0.0f;
             for (const int rows : {128, 192})
                 for (const int sp : {1, 2, 4}) {

@@ -22,6 +22,10 @@ pytestmark = pytest.mark.gpu
     (sg.F16, 1920, 2000, 130, "gemm lds w=8 kg=2 bn=128 rows=128"),         # 30 stages
     (sg.F16, 4224, 12290, 380, "gemm wide w=12 kg=1 bn=128 rg=1 split=2 lds"),  # 384-row tiles, 33 stages a split
     (sg.BF16, 128, 24576, 500, "gemm wide w=12 kg=1 bn=128 rg=1 split=1 lds"),  # two stages in all
+    (sg.F16, 512, 9001, 1000, "gemm lds w=8 kg=2 bn=128 rows="),            # short K: 568 tiles of 128 x 128, a last round of 56
+    (sg.BF16, 896, 28672, 300, "gemm lds w=8 kg=2 bn=128 rows="),           # 672 of them
+    (sg.F16, 640, 9001, 1500, "gemm w=4 kg=1 bn=128"),                      # 852: a last round two thirds full
+    (sg.F16, 384, 9001, 1000, "gemm w=4 kg=1 bn=128"),                      # K below 512
 ], ids=lambda v: str(v).replace(" ", "_"))
 def test_gemm_lds(hip, dtype, K, M, N, form):
     dev, st = hip
