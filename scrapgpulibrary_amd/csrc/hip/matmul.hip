@@ -692,20 +692,18 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     const Slice slc = slice_of(L.a, sl);
     // the wave's matrix (several when weights share x)
     const int64_t grow = tm * BMT + 32 * RG * wave; // packed: the wave's first row over all matrices
-    // (float weights: its entries by index, and only where there are several: with pick3 BF16 2000x640
-    // took 13.87 us at 16 tokens and 14.80 at 64, against 13.36 and 14.36)
-    constexpr bool FW = DT == F16 || DT == BF16;
-    const bool one = GA || (FW && L.nmat == 1);
+    // (its entries by index, and only where there are several: with pick3 BF16 2000x640 took 13.87 us at 16
+    // tokens against 13.36, Q4_K 69x768 at 129 18.27 against 17.93, Q6_K 20000x1024 at 12 14.46 against 14.04)
+    const bool one = GA || L.nmat == 1;
     const int mj = one ? 0
                  : L.packed ? min(L.nmat - 1, grow >= L.mo[1] ? (grow >= L.mo[2] ? 2 : 1) : 0)
                             : (tm >= L.mt[1] ? (tm >= L.mt[2] ? 2 : 1) : 0);
-    const auto entry = [&](const auto * v) __attribute__((always_inline)) { return FW ? v[mj] : pick3(v, mj); };
-    const uint8_t * w = GA ? L.a.w : FW && !one ? entry(L.wm) : (FW ? L.a.w : entry(L.wm)) + slice_w(L.a, slc);
+    const uint8_t * w = GA ? L.a.w : one ? L.a.w + slice_w(L.a, slc) : L.wm[mj];
     const int64_t K = L.a.K, nb = L.a.nb;
-    const int64_t M = one ? L.a.M : entry(L.Mm);
+    const int64_t M = one ? L.a.M : L.Mm[mj];
     int64_t N = L.a.N;
     int64_t n0 = tn * BN;
-    const int64_t m0 = GA ? grow : L.packed ? grow - entry(L.mo) : (tm - entry(L.mt)) * BMT + 32 * RG * wave;
+    const int64_t m0 = GA ? grow : L.packed ? grow - L.mo[mj] : (tm - L.mt[mj]) * BMT + 32 * RG * wave;
     int32_t * ga_rows = reinterpret_cast<int32_t *>(lds_mm + KG * 2 * BN * BK); // GA: x row of tile token n
     int64_t * ga_y = reinterpret_cast<int64_t *>(ga_rows + BN);               // GA: its y element offset
     int32_t ga_cnt = BN;                                                      // GA: the tile's pairs
@@ -974,11 +972,11 @@ __global__ __launch_bounds__(64 * W, occupancy_of(DT, BN, RG, W)) void k_matmul(
     float * y;
     int64_t ys1;
     if (L.split == 1) {
-        y = GA ? L.a.y : FW && !one ? entry(L.ym) : (FW ? L.a.y : entry(L.ym)) + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3;
-        ys1 = one ? L.a.y_s1 : entry(L.ys1m);
+        y = GA ? L.a.y : one ? L.a.y + slc.i2 * L.a.y_s2 + slc.i3 * L.a.y_s3 : L.ym[mj];
+        ys1 = one ? L.a.y_s1 : L.ys1m[mj];
     } else {
         const int64_t mt_all = L.mo[L.nmat]; // the partials' row length: all matrices' rows
-        y = L.part + ((uint64_t) split * slices + (uint64_t) sl) * N * mt_all + entry(L.mo);
+        y = L.part + ((uint64_t) split * slices + (uint64_t) sl) * N * mt_all + L.mo[mj];
         ys1 = mt_all;
     }
     const float * xs = L.xs + (uint64_t) sl * N;
