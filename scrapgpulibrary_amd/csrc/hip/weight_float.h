@@ -15,46 +15,6 @@ __device__ __forceinline__ uint4 ld16_nt(const uint8_t * p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// 8 weights of one row as f32 (addresses 16-byte aligned): 8 consecutive ones, or for F32 also two
-// separate groups of 4
-template <int WT> struct WLoad;
-template <> struct WLoad<F32> {
-    uint4 u, v;
-    __device__ void load(const uint8_t * p, const uint8_t * p2) {
-        u = ld16_nt(p);
-        v = ld16_nt(p2);
-    }
-    __device__ void load(const uint8_t * p) { load(p, p + 16); }
-    __device__ void to_f32(float * o) const {
-        o[0] = __uint_as_float(u.x), o[1] = __uint_as_float(u.y), o[2] = __uint_as_float(u.z), o[3] = __uint_as_float(u.w);
-        o[4] = __uint_as_float(v.x), o[5] = __uint_as_float(v.y), o[6] = __uint_as_float(v.z), o[7] = __uint_as_float(v.w);
-    }
-};
-template <> struct WLoad<F16> {
-    uint4 q;
-    __device__ void load(const uint8_t * p) { q = ld16_nt(p); }
-    __device__ void to_f32(float * o) const {
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[2 * i] = __half2float(__ushort_as_half((unsigned short) (w[i] & 0xFFFFu)));
-            o[2 * i + 1] = __half2float(__ushort_as_half((unsigned short) (w[i] >> 16)));
-        }
-    }
-};
-template <> struct WLoad<BF16> {
-    uint4 q;
-    __device__ void load(const uint8_t * p) { q = ld16_nt(p); }
-    __device__ void to_f32(float * o) const {
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[2 * i] = __uint_as_float(w[i] << 16);
-            o[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-        }
-    }
-};
-
 // 16 bytes of weights (4 F32 or 8 F16 / BF16) as f32
 template <int WT>
 __device__ __forceinline__ void widen16(uint4 q, float * o) {
@@ -72,5 +32,23 @@ __device__ __forceinline__ void widen16(uint4 q, float * o) {
         }
     }
 }
+
+// 8 consecutive weights of one row as f32 (p 16-byte aligned)
+template <int WT> struct WLoad {
+    uint4 q;
+    __device__ void load(const uint8_t * p) { q = ld16_nt(p); }
+    __device__ void to_f32(float * o) const { widen16<WT>(q, o); }
+};
+template <> struct WLoad<F32> {
+    uint4 u, v;
+    __device__ void load(const uint8_t * p) {
+        u = ld16_nt(p);
+        v = ld16_nt(p + 16);
+    }
+    __device__ void to_f32(float * o) const {
+        widen16<F32>(u, o);
+        widen16<F32>(v, o + 4);
+    }
+};
 
 } // namespace sgk
