@@ -1250,7 +1250,7 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemm_w(MmArgs L) {
     // (GA: a tile of at most 32 pairs runs a loop of its own without the second token fragment's
     // MFMAs; a branch around each of them cut every k-step into basic blocks that the compiler
     // cannot schedule across: with the tile table and the earlier weights, gate, up and down of 128
-    // Q4_K experts of 768 x 2048, 8 of them per token, 512 tokens, 157 -> 150 us)
+    // Q4_K experts of 768 x 2048, 8 of them per token, 512 tokens, 163.6 -> 156.2 us)
     if (GA && half_tile) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, NF>{});
     // acc[q][v], lane (j, h): token n0 + 32q + 8 (v / 4) + 4h + v % 4, weight row m0 + j
@@ -1989,9 +1989,10 @@ MmConfig config_of(const MatArgs & a, int cu_count, bool lean) {
         const int64_t tiles = tm * ((a.N + c.bn - 1) / c.bn) * slices;
         // the split with the least estimated time: rounds of cu_count work-groups x (stages per
         // split + 4, a work-group's fixed cost in stages), the fewer splits on a tie, every split
-        // >= 8 stages (F16, 128-token tiles, measured on 256 CUs: 12288x4096 at 128 tokens, 96
-        // tiles, 55.7 / 64.6 / 56.3 / 62.4 us at 2 / 3 / 4 / 8 splits; 4096x4096, 32 tiles, 31 us
-        // at 8 against 36 at 4; 12288x4096 at 256 tokens 78 us unsplit against 80-87 split)
+        // >= 8 stages (F16, 64-token tiles, measured on 256 CUs: 12288x4096 at 64 tokens, 96 tiles,
+        // 32.4 / 35.5 / 39.0 us at 2 / 4 / 8 splits; 20000x4096 at 33, 157 tiles, 48.3 / 41.2 / 45.1
+        // at 2 / 3 / 4; 4096x4096 at 32, 32 tiles, 29.0 / 21.8 at 2 / 4, and 18.9 at 8 splits of 4
+        // stages, which the least of 8 leaves out)
         c.split = 1;
         if (env_split > 0) {
             c.split = (int) std::max<int64_t>(1, std::min<int64_t>(std::min(env_split, 8), (stages + 3) / 4));
