@@ -17,7 +17,8 @@
 // larger; F16 4096x4096 at 8 columns 9.2e-8 against 1.06e-7, 12288x2056 at 300 8.5e-8 against 9.3e-8,
 // F32 128x2048 at 512 8.8e-8 against 9.2e-8, 512x512 at 1024 7.9e-8 against 8.2e-8, 512x8192 at 2048
 // 1.10e-7 against 1.27e-7; with the waves' sums added in f32 it was up to 6% above it at K of 500 to
-// 2100).
+// 2100; k_mvq at K of 130 to 250, whose steps fill one wave and part of a second, within 0.4% of it;
+// k_mmf at K of 8, where nothing follows the tree of 8 products, 5.1e-8 against 4.5e-8).
 #include "kernels.h"
 #include "weight_float.h"
 
@@ -247,8 +248,10 @@ __global__ __launch_bounds__(64 * W) void k_mmf(MmfArgs A) {
     // descending order: an MFMA adds its 4 products one after the other, so the first is rounded four
     // times and the last once. Random data do not care; with large activations in a step's first part
     // this order has the smaller error, F16 64x64 6.3e-8 against 7.0e-8. F32 keeps the ascending order,
-    // 128x2048 at 512 columns 9.6 us against 9.8.)
-    const int g = WT == F32 ? q : 3 - q, o0 = WT == F32 ? 4 * g : 8 * g, o1 = WT == F32 ? 16 + 4 * g : 8 * g + 4;
+    // 128x2048 at 512 columns 9.6 us against 9.8, but for short K, where the sums that follow do not
+    // make up for it: 1270x16 at 471 columns 5.3e-8 in the vector kernel, 5.7e-8 ascending, 5.2e-8
+    // descending; 115x120 at 449 7.25e-8 and 7.33e-8 ascending.)
+    const int g = WT == F32 && K >= 256 ? q : 3 - q, o0 = WT == F32 ? 4 * g : 8 * g, o1 = WT == F32 ? 16 + 4 * g : 8 * g + 4;
     struct Raw {
         uint4 w[R][S][WT == F32 ? 2 : 1];
         float4 x[C][S][2];

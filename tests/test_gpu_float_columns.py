@@ -105,7 +105,8 @@ def test_float_columns_non_finite(hip, dtype, K, M, N):
 
 
 @pytest.mark.parametrize("dtype,K,M,N", [(sg.BF16, 520, 4096, 5), (sg.F16, 4096, 3072, 8), (sg.F16, 1000, 1000, 64), (sg.BF16, 2056, 1500, 40),
-                                         (sg.F32, 512, 512, 1100), (sg.F32, 1024, 300, 128), (sg.F16, 64, 1000, 30)], ids=lambda v: str(v))
+                                         (sg.F32, 512, 512, 1100), (sg.F32, 1024, 300, 128), (sg.F16, 64, 1000, 30),
+                                         (sg.F32, 16, 1270, 471), (sg.F32, 40, 1500, 94), (sg.F32, 120, 1150, 449)], ids=lambda v: str(v))
 def test_float_columns_error(hip, dtype, K, M, N):
     """The error against 64-bit products is no larger than the vector kernel's (1 and 2 columns per call),
     on activations with outlier channels."""
