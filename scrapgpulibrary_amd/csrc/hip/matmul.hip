@@ -502,10 +502,12 @@ __device__ __forceinline__ int64_t slice_w(const MatArgs & a, const Slice & c) {
 __device__ __forceinline__ uint32_t row_slice(int64_t row, int64_t n) { // the slice of x row `row`
     return row < n ? 0 : (uint32_t) row / (uint32_t) n;
 }
-// the first stage of a split (K in groups of 4 stages; split = n: K's end, or up to 3 past it)
+// the first stage of a split (K in groups of 4 stages; split = n: K's end, or up to 3 past it). Divided in
+// 64 bits, behind the branch: in 32 bits the tiled GEMM takes 4 more registers and Q8_0 507x2208 at 144
+// tokens 27.0 us against 26.7, 1433x5472 at 225 36.3 against 36.1
 __device__ __forceinline__ int64_t split_start(int64_t groups, int split, int n) {
     if (split == 0) return 0;
-    return 4 * (split == n ? groups : (int64_t) ((uint32_t) groups * (uint32_t) split / (uint32_t) n));
+    return 4 * (split == n ? groups : groups * split / n);
 }
 struct TileOf {
     int64_t tm, tn;
